@@ -75,6 +75,7 @@ struct Phase {
   int os, oy0, ox0;       // output scatter: y row = oy * os + oy0, column = ox * os + ox0
   int woff;               // offset of this phase's [P][K] weights (floats)
   int ky0, kx0;           // grad input read straight from w: the phase's first filter tap
+  int soff, snkb;         // split tile: the phase's first 16-byte unit of the packed filter, and its K-blocks
   FastDiv div_ohw, div_ow, div_kk, div_kw;
 };
 
@@ -100,7 +101,9 @@ struct GatherArgs {
   int wplace;            // tap-major order with the filter read in place: 1 forward, A[co][(tap, ci)] from
                          //   w[co][ci][ky][kx]; 2 grad input, A[ci][(a', b', co)] from w[co][ci][ky][kx] through the
                          //   phase's flip map (ky = ky0 + s (KH - 1 - a')); 0 the [P][K] filter at w (re-packed)
-  uint32_t w_rowst, w_cst;  // wplace: bytes between A rows and between consecutive channels of one tap
+  uint32_t w_rowst, w_cst, w_tst;  // wplace: bytes between A rows, consecutive channels of one tap, and taps
+  const uint32_t* wsplit;  // split tile: the filter in split_pack_kernel's layout
+  uint32_t wsplit_bytes;
   float* part;           // split K: raw partials [slices][N][P][YH][YW], else null (epilogue writes y)
   int64_t part_stride;   // elements per slice
   int nhwc;              // channels-last source [N][H][W][C] and output [N][YH][YW][P] (partials likewise)
@@ -484,7 +487,7 @@ __device__ __forceinline__ void gather_tile(const GatherArgs& a, const int bx, c
           tkx = a.wplace == 1 ? nkx : ph.kx0 + a.s * (KW - 1 - nkx);
         }
         // nc0 is the channel of this thread's first k-row (k0 + rbase, one tap per block): the block starts rbase back
-        const uint32_t sb = (uint32_t)(nc0 - rbase) * a.w_cst + (uint32_t)((tky * a.ks + tkx) * 4);
+        const uint32_t sb = (uint32_t)(nc0 - rbase) * a.w_cst + (uint32_t)(tky * a.ks + tkx) * a.w_tst;
 #pragma unroll
         for (int i = 0; i < AR4; ++i)
           ra4[set][i] = make_float4(bload(wr, aoff4[i], sb), bload(wr, aoff4[i], sb + a.w_cst),
@@ -693,6 +696,362 @@ __device__ __forceinline__ void gather_tile(const GatherArgs& a, const int bx, c
     row_epilogue<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane, lds + wave * row_epi_floats<WQ>());
   else
     gather_epilogue<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane, zs);
+}
+
+// ---- split-bf16 gather tiles --------------------------------------------------------------------------------------
+// Tile 1 runs fp32 products on the bf16 matrix cores. Each float is split into three bf16 terms x = h + m + l (round
+// to nearest each time: 24 significant bits, so the split is exact but for terms below the smallest bf16 subnormal),
+// and a product keeps the six partial products above 2^-24 of it: hh, hm + mh, mm, hl + lh (those left out are at
+// most 2^-26 of hh each). bf16 products are exact in the matrix core's fp32 accumulator. Six
+// v_mfma_f32_16x16x32_bf16 (1950 TFLOP/s dense here on random data) do the work of eight v_mfma_f32_16x16x4_f32
+// (146 TFLOP/s): 2.2 times the rate.
+// Accuracy: each 32-deep K-block is summed from zero, smallest partial products first, and added to the running sum
+// with one fp32 add, so the running sum is rounded once per 32 products, where the fp32 instruction rounds it per
+// product. Against float64 sums of random products the relative error is 0.9e-7 at K 576 and 2.4e-7 at K 4608; the
+// fp32 MFMA chain has 3.0-4.4e-7 and 0.9-1.2e-6.
+// Range: a value whose split overflows (infinite, NaN, or within 2^-9 of the largest float), or an overflowing sum,
+// leaves a non-finite accumulator; inputs so small that their low terms underflow leave only tiny ones. A tile that
+// holds a non-finite sum, or whose largest sum is below 2^-60 and not zero, is computed again by the fp32 tile
+// (split_redo), so such inputs give what the fp32 instructions give.
+typedef __bf16 omt_bf16x8 __attribute__((ext_vector_type(8)));
+
+// Terms h, m, l of two floats, each pair packed as two bf16 (x in the low half).
+__device__ __forceinline__ void split_bf16(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
+  // (through the conversion in C++ the compiler converts some terms twice, once packed and once alone)
+  const auto pack = [](float a, float b) {
+    uint32_t r;
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+  };
+  const auto lo = [](uint32_t v) { return __builtin_bit_cast(float, v << 16); };
+  const auto hi = [](uint32_t v) { return __builtin_bit_cast(float, v & 0xffff0000u); };
+  h = pack(x, y);
+  const float x1 = x - lo(h), y1 = y - hi(h);
+  m = pack(x1, y1);
+  l = pack(x1 - lo(m), y1 - hi(m));
+}
+
+// A K-block of 32 k of R rows is staged as 16-byte units of 8 k of one row and one term, unit (term z, k group g,
+// row r) at (4 z + g) R + r: the 16 rows that one b128 read of an MFMA operand touches are contiguous, and so are the
+// rows that a wave writes, so both run without bank conflicts.
+constexpr int kSplitBK = 32, kSplitRun = 16;  // K-block; channels per tap run of the tap-major order
+constexpr int kSplitNT = 512;                 // threads of a workgroup (one per CU: two waves per SIMD)
+
+// The filter, packed for the split tile: for each phase, tile of BP rows and K-block, the K-block's units in LDS
+// order, rows past P and k past K zero. One thread per (row, 8 k): three units.
+template <int BP>
+__global__ void __launch_bounds__(256) split_pack_kernel(const GatherArgs a, uint4* __restrict__ out, int nunits) {
+  const int u = blockIdx.x * 256 + threadIdx.x;
+  if (u >= nunits) return;
+  int f = 0;
+  while (f + 1 < a.nphase && u * 3 >= a.ph[f + 1].soff) ++f;
+  const Phase& ph = a.ph[f];
+  const int r = u - ph.soff / 3, row = r % BP, g = r / BP % 4, blk = r / (4 * BP);  // blk = ptile nkb + kb
+  const int pt = blk / ph.snkb, k0 = (blk - pt * ph.snkb) * kSplitBK + 8 * g, p = pt * BP + row;
+  float v[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int k = k0 + e;
+    uint32_t off;  // bytes; the filter is below 2 GiB
+    if (a.wplace) {
+      const int tap = (int)fdiv((uint32_t)k, a.div_c), c = k - tap * a.C;
+      const int ay = (int)fdiv((uint32_t)tap, ph.div_kw), ax = tap - ay * ph.KW;
+      const int ky = a.wplace == 1 ? ay : ph.ky0 + a.s * (ph.KH - 1 - ay);
+      const int kx = a.wplace == 1 ? ax : ph.kx0 + a.s * (ph.KW - 1 - ax);
+      off = (uint32_t)p * a.w_rowst + (uint32_t)c * a.w_cst + (uint32_t)(ky * a.ks + kx) * a.w_tst;
+    } else if (a.wdirect) {
+      const int co = (int)fdiv((uint32_t)k, ph.div_kk), tt = k - co * ph.KH * ph.KW;
+      const int ap = (int)fdiv((uint32_t)tt, ph.div_kw), bp = tt - ap * ph.KW;
+      const int ky = ph.ky0 + a.s * (ph.KH - 1 - ap), kx = ph.kx0 + a.s * (ph.KW - 1 - bp);
+      off = (uint32_t)((((co * a.P + p) * a.ks + ky) * a.ks + kx) * 4);
+    } else {
+      off = (uint32_t)((ph.woff + p * ph.K + k) * 4);
+    }
+    v[e] = p < a.P && k < ph.K ? a.w[off / 4] : 0.f;
+  }
+  uint32_t h[4], m[4], l[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) split_bf16(v[2 * e], v[2 * e + 1], h[e], m[e], l[e]);
+  uint4* const o = out + ph.soff + (int64_t)blk * 12 * BP + g * BP + row;
+  o[0] = make_uint4(h[0], h[1], h[2], h[3]);
+  o[4 * BP] = make_uint4(m[0], m[1], m[2], m[3]);
+  o[8 * BP] = make_uint4(l[0], l[1], l[2], l[3]);
+}
+
+// Whether a workgroup's finished sums call for the fp32 tile (see above), the same answer in every thread. Uses a
+// dword of LDS per wave at `flags` that no wave still reads; returns after a barrier, with `flags` free again.
+template <int TI, int TJ, int NW>
+__device__ __forceinline__ bool split_redo(const omt_f32x4 (&acc)[TI][TJ], int wave, int lane, uint32_t* flags) {
+  uint32_t m = 0;
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m = max(m, __builtin_bit_cast(uint32_t, acc[i][j][r]) & 0x7fffffffu);
+  constexpr uint32_t kTiny = (127u - 60u) << 23;  // 2^-60
+  const uint32_t bits = (__ballot(m >= 0x7f800000u) ? 1u : 0u) | (__ballot(m >= kTiny) ? 2u : 0u) |
+                        (__ballot(m != 0) ? 4u : 0u);
+  if (lane == 0) flags[wave] = bits;
+  __syncthreads();
+  uint32_t all = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) all |= flags[w];
+  __syncthreads();
+  return (all & 1u) || (all & 6u) == 4u;
+}
+
+// Units between consecutive k groups of the staged source: channels last, four more than its rows, so that the four
+// groups that a quad of lanes writes for one pixel fall on disjoint banks.
+template <int BQ, int MODE>
+constexpr int split_bstride() { return BQ + (MODE == kNhwc ? 4 : 0); }
+template <int BP, int BQ, int MODE>
+constexpr int split_lds_units() { return 12 * (BP + split_bstride<BQ, MODE>()); }  // of one buffer
+
+// One workgroup's split-bf16 tile: gather_tile's source loaders (kGeneric, kTapMajor, kNhwc), plans and epilogues. The
+// filter comes packed (split_pack_kernel) and goes to LDS directly; the source is split as it is staged. K-blocks are
+// two runs of 16 k: in the tap-major orders a run is 16 channels of one tap (C % 16 == 0), so that the K order does
+// not depend on whether C is a multiple of 32. Two LDS buffers: while the MFMAs of K-block b run, the wave splits and
+// stores its part of b + 1 between them, b + 1's filter is on its way to LDS, and b + 2's source is being loaded.
+template <int BP, int BQ, int WP, int WQ, int MODE>
+__device__ __forceinline__ void gather_split_tile(const GatherArgs& a, const int bx, const int by, const int bz,
+                                                  uint4* __restrict__ lds) {
+  constexpr int NT = kSplitNT, NW = NT / 64, BK = kSplitBK, RUN = kSplitRun;
+  constexpr int WGQ = BQ / WQ;
+  static_assert((BP / WP) * (BQ / WQ) == NW && WP % 16 == 0 && WQ == 64 && BQ == NT / 2, "tile shape");
+  constexpr int TI = WP / 16, TJ = WQ / 16;
+  constexpr int BS = split_bstride<BQ, MODE>(), BUF = split_lds_units<BP, BQ, MODE>();
+
+  const int zs = bz / a.nphase;  // K slice
+  const Phase ph = a.ph[bz - zs * a.nphase];
+  const int q0 = bx * BQ, p0 = by * BP;
+  if (q0 >= ph.Q) return;  // this phase has fewer pixel tiles than the largest one
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wp = wave / WGQ, wq = wave % WGQ;
+  const int KH = ph.KH, KW = ph.KW, K = ph.K, KK = KH * KW;
+  const int H = a.H, W = a.W, HW = H * W, C = a.C;
+  const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, a.x_bytes);
+
+  // This thread's part of a K-block of the source: k rbase .. rbase + 15 of pixel t % BQ, or, channels last, k 8 cg ..
+  // 8 cg + 7 of pixels t / 4 and t / 4 + 128 (four lanes read one pixel's contiguous 128 bytes).
+  // lb0: byte offset of x[n][0][iy][ix] (channels last: of the first of its channels of the pixel)
+  constexpr int NPX = MODE == kNhwc ? 2 : 1;
+  const int run = MODE == kNhwc ? (t & 3) >> 1 : __builtin_amdgcn_readfirstlane(t / BQ);
+  const int rbase = RUN * run, cg = t & 3;
+  int iy[NPX], ix[NPX];
+  uint32_t lb0[NPX];
+#pragma unroll
+  for (int j = 0; j < NPX; ++j) {
+    const int q = q0 + (MODE == kNhwc ? t / 4 + 128 * j : t % BQ);
+    iy[j] = ix[j] = -(1 << 28);  // pixels past Q gather nothing
+    lb0[j] = kOOB;
+    if (q < ph.Q) {
+      const uint32_t ohw = (uint32_t)(ph.OH * ph.OW);
+      const uint32_t n = fdiv((uint32_t)q, ph.div_ohw), r = (uint32_t)q - n * ohw;
+      const uint32_t oy = fdiv(r, ph.div_ow), ox = r - oy * (uint32_t)ph.OW;
+      iy[j] = (int)oy * ph.S - ph.PH;
+      ix[j] = (int)ox * ph.S - ph.PW;
+      lb0[j] = MODE == kNhwc ? (uint32_t)((((int)n * H + iy[j]) * W + ix[j]) * C * 4 + 32 * (cg & 1))
+                             : (uint32_t)(((int)n * C * HW + iy[j] * W + ix[j]) * 4);
+    }
+  }
+
+  const int kbeg = zs * a.kslice, kend = min(K, kbeg + a.kslice);
+  const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;  // an empty slice still writes its (zero) tile
+  // tap-major orders: the tap (rky, rkx) and first channel rc of this thread's run of the next K-block gload reads
+  int rc = 0, rky = 0, rkx = 0;
+  if constexpr (MODE != kGeneric) {
+    const uint32_t kb = (uint32_t)(kbeg + rbase);
+    const int tap = (int)fdiv(kb, a.div_c);
+    rc = (int)kb - tap * C;
+    rky = (int)fdiv((uint32_t)tap, ph.div_kw);
+    rkx = tap - rky * KW;
+  }
+
+  float rb[2][RUN];  // two register sets: source loads two K-blocks ahead of the MFMAs
+  auto gload = [&](int k0, const int set) {
+    if constexpr (MODE == kGeneric) {
+      const uint32_t kb = (uint32_t)(k0 + rbase);
+      int c = (int)fdiv(kb, ph.div_kk);
+      const uint32_t rr = kb - (uint32_t)c * (uint32_t)KK;
+      int ky = (int)fdiv(rr, ph.div_kw);
+      int kx = (int)rr - ky * KW;
+#pragma unroll
+      for (int e = 0; e < RUN; ++e) {
+        const bool ok = (k0 + rbase + e < K) & ((unsigned)(iy[0] + ky) < (unsigned)H) & ((unsigned)(ix[0] + kx) < (unsigned)W);
+        rb[set][e] = bload(xr, ok ? lb0[0] + (uint32_t)((c * HW + ky * W + kx) * 4) : kOOB, 0);
+        if (++kx == KW) {
+          kx = 0;
+          if (++ky == KH) {
+            ky = 0;
+            ++c;
+          }
+        }
+      }
+      return;
+    }
+    const bool kin = k0 + rbase < K;  // the second half of an odd last block is past K
+    if constexpr (MODE == kNhwc) {
+      const uint32_t toff = (uint32_t)(((rky * W + rkx) * C + rc) * 4);
+#pragma unroll
+      for (int j = 0; j < NPX; ++j) {
+        const bool ok = kin & ((unsigned)(iy[j] + rky) < (unsigned)H) & ((unsigned)(ix[j] + rkx) < (unsigned)W);
+        const uint32_t off = ok ? lb0[j] + toff : kOOB;
+        const float4 v0 = bload4(xr, off, 0), v1 = bload4(xr, off, 16);
+        float* const d = &rb[set][8 * j];
+        d[0] = v0.x, d[1] = v0.y, d[2] = v0.z, d[3] = v0.w, d[4] = v1.x, d[5] = v1.y, d[6] = v1.z, d[7] = v1.w;
+      }
+    } else {
+      const bool ok = kin & ((unsigned)(iy[0] + rky) < (unsigned)H) & ((unsigned)(ix[0] + rkx) < (unsigned)W);
+      const uint32_t voff = ok ? lb0[0] + (uint32_t)((rky * W + rkx) * 4) : kOOB;
+#pragma unroll
+      for (int e = 0; e < RUN; ++e) rb[set][e] = bload(xr, voff, (uint32_t)((rc + e) * HW * 4));
+    }
+    rc += BK;  // the next K-block's run; 32 channels on may cross two taps (C of 16)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const bool over = rc >= C;
+      rc -= over ? C : 0;
+      rkx += over;
+      const bool wrap = rkx == KW;
+      rkx = wrap ? 0 : rkx;
+      rky += wrap;
+    }
+  };
+  constexpr int NLOADS = MODE == kNhwc ? 4 : RUN;  // of one gload
+
+  // The filter's K-block kb (of the slice's first), 1 KB per instruction: BP 12 units of 16 bytes.
+  const omt_u32x4 wr = rsrc_words(a.wsplit, a.wsplit_bytes);
+  constexpr int AKB = BP * 12 / 64;  // 1 KB pieces
+  const uint32_t alds = lds_addr(reinterpret_cast<const float*>(lds));
+  const uint32_t asrc = (uint32_t)((ph.soff + (by * ph.snkb + kbeg / BK) * 12 * BP) * 16);
+  auto aload = [&](int it, const int buf) {
+#pragma unroll
+    for (int i = 0; i < (AKB + NW - 1) / NW; ++i) {
+      const int c = wave + NW * i;
+      if (AKB % NW == 0 || c < AKB)
+        lds_load_b128s(wr, alds + (uint32_t)(buf * BUF * 16 + c * 1024), (uint32_t)(lane * 16),
+                       asrc + (uint32_t)(it * 12 * BP * 16 + c * 1024));
+    }
+  };
+
+  // A quarter of this thread's source values: split four k, and store each eight as three units.
+  uint32_t sh[4], sm[4], sl[4];
+  auto sstore = [&](const int quarter, const int set, const int buf) {
+    const int e = 4 * quarter, u = 2 * (quarter & 1);
+    split_bf16(rb[set][e], rb[set][e + 1], sh[u], sm[u], sl[u]);
+    split_bf16(rb[set][e + 2], rb[set][e + 3], sh[u + 1], sm[u + 1], sl[u + 1]);
+    if (quarter & 1) {
+      const int g = MODE == kNhwc ? cg : rbase / 8 + quarter / 2;
+      const int row = MODE == kNhwc ? t / 4 + 128 * (quarter / 2) : t % BQ;
+      uint4* const o = lds + buf * BUF + 12 * BP + g * BS + row;
+      o[0] = make_uint4(sh[0], sh[1], sh[2], sh[3]);
+      o[4 * BS] = make_uint4(sm[0], sm[1], sm[2], sm[3]);
+      o[8 * BS] = make_uint4(sl[0], sl[1], sl[2], sl[3]);
+    }
+  };
+
+  omt_f32x4 acc[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[i][j] = omt_f32x4{0.f, 0.f, 0.f, 0.f};
+  // Lane group grp supplies k = 8 grp .. 8 grp + 7 of both operands; the accumulator layout is that of the 16x16x4
+  // fp32 instruction.
+  const int la = wp * WP + (lane & 15), lb = wq * WQ + (lane & 15), grp = lane >> 4;
+
+  // End of a step: this wave's LDS writes and its filter loads (issued before the NLOADS source loads in flight) done.
+  auto sync = [&]() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(NLOADS) & ~0xF00);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  aload(0, 0);
+  gload(kbeg, 0);
+#pragma unroll
+  for (int v = 0; v < 4; ++v) sstore(v, 0, 0);
+  gload(kbeg + BK, 1);
+  sync();
+  omt_bf16x8 av[3][TI], bv[2][3];
+  omt_f32x4 s[2][TI];  // the K-block's sums of column tiles j and j - 1
+#pragma unroll
+  for (int i = 0; i < TI; ++i) s[(TJ - 1) & 1][i] = omt_f32x4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](int it, auto setc) {
+    constexpr int S = decltype(setc)::value;  // it & 1
+    constexpr int za[6] = {2, 0, 1, 1, 0, 0}, zb[6] = {0, 2, 1, 0, 1, 0};  // smallest partial products first
+    const auto frag = [&](int unit) { return __builtin_bit_cast(omt_bf16x8, lds[S * BUF + unit]); };
+    const auto bread = [&](int j, int z) { return frag(12 * BP + (4 * z + grp) * BS + lb + 16 * j); };
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+#pragma unroll
+      for (int i = 0; i < TI; ++i) av[za[z]][i] = frag((4 * za[z] + grp) * BP + la + 16 * i);
+      bv[0][zb[z]] = bread(0, zb[z]);
+    }
+    aload(it + 1, S ^ 1);
+    gload(kbeg + (it + 2) * BK, S);
+    // Column tile j's MFMAs run beside the additions and a quarter of the staging of the tile before.
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+#pragma unroll
+      for (int z = 0; z < 3; ++z)
+        if (j + 1 < TJ) bv[(j + 1) & 1][zb[z]] = bread(j + 1, zb[z]);
+#pragma unroll
+      for (int i = 0; i < TI; ++i) s[j & 1][i] = omt_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int z = 0; z < 6; ++z)
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+          s[j & 1][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[za[z]][i], bv[j & 1][zb[z]], s[j & 1][i], 0, 0, 0);
+      if (j > 0) sstore(j - 1, S ^ 1, S ^ 1);
+      if (j == TJ - 1) sstore(j, S ^ 1, S ^ 1);
+#pragma unroll
+      for (int i = 0; i < TI; ++i) acc[i][(j + TJ - 1) % TJ] += s[(j + 1) & 1][i];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    sync();
+  };
+  // Whole pairs of steps in the loop and an odd last one after it: a conditional second step merges two load histories
+  // at the loop head, where the compiler then waits for every load in flight.
+  int it = 0;
+  for (; it + 1 < nk; it += 2) {
+    step(it, std::integral_constant<int, 0>{});
+    step(it + 1, std::integral_constant<int, 1>{});
+  }
+  if (it < nk) step(it, std::integral_constant<int, 0>{});
+#pragma unroll
+  for (int i = 0; i < TI; ++i) acc[i][TJ - 1] += s[(TJ - 1) & 1][i];
+
+  static_assert(NW * row_epi_floats<WQ>() <= 4 * BUF && gather_lds_floats<64, 128, 16>() <= 4 * BUF,
+                "epilogue and fp32 tile fit the LDS");
+  float* const fl = reinterpret_cast<float*>(lds);
+  if (split_redo<TI, TJ, NW>(acc, wave, lane, reinterpret_cast<uint32_t*>(lds))) {
+    // the fp32 tile is the work of four waves; a barrier waits for the waves that have not ended
+    if (wave >= 4) return;
+    constexpr int FQ = BQ / 128, FP = BP / 64, FMODE = MODE == kTapMajor ? kTapInPlace : MODE;
+#pragma unroll 1
+    for (int f = 0; f < FP * FQ; ++f) {
+      gather_tile<64, 128, 32, 64, 16, FMODE, false, 2>(a, bx * FQ + f % FQ, by * FP + f / FQ, bz, fl);
+      __syncthreads();
+    }
+    return;
+  }
+  if constexpr (MODE == kNhwc)
+    gather_epilogue_nhwc<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane, zs);
+  else if (a.d2s && !a.part)
+    d2s_epilogue<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane);
+  else if (a.rows)
+    row_epilogue<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane, fl + wave * row_epi_floats<WQ>());
+  else
+    gather_epilogue<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane, zs);
+}
+
+template <int BP, int BQ, int WP, int WQ, int MODE>
+__global__ void __launch_bounds__(kSplitNT, 2) conv_gather_split_kernel(const GatherArgs a) {
+  __shared__ __attribute__((aligned(16))) uint4 lds[2 * split_lds_units<BP, BQ, MODE>()];
+  const TileId t = xcd_block_tile(kTileGroup);
+  gather_split_tile<BP, BQ, WP, WQ, MODE>(a, t.x, t.y, t.z, lds);
 }
 
 // 1x1, stride 1, unpadded convolutions (and their grad input, a 1x1 convolution with the transposed filter) with a
@@ -1859,13 +2218,18 @@ __global__ void __launch_bounds__(256) fold_bn_kernel(int co, int per_out, const
 
 // ---- tile selection and launch ----------------------------------------------------------------------------------
 
+constexpr int64_t kCUs = 256;
+
 struct Tile {
   int bp, bq, wp, wq;
   float eff;    // relative MFMA efficiency of the wave tile (operand reuse)
   int bk = 16;  // K-block (gather kernels)
   int ns = 0;   // > 0: direct global -> LDS loads into an ns-stage ring (tap-major order; else the staged kernel)
+  int split = 0;  // 1: conv_gather_split_kernel (bp by the output channels: tile_bp)
   int stream = 0;  // 1x1 stride-1 convolutions only: 1 conv1x1_stream_kernel (runs of pixel tiles per workgroup),
                    // 2 conv1x1_wst_kernel (K of 64 or 128, the filter held in registers)
+  // channels per tap run of the tap-major K orders: C is a multiple of it
+  constexpr int run() const { return split ? kSplitRun : bk; }
 };
 
 // Picks the tile with the smallest estimated makespan: rounds of `slots` concurrent workgroups times the padded
@@ -1892,13 +2256,13 @@ static int pick_tile(const Tile (&tiles)[N], int64_t P, int64_t Q, int64_t z, in
 // 64x64 input: 64 channels over 8192 pixels) twice the workgroups of the 64 x 64 tile, so that every CU holds one
 // without a K split.
 static const Tile kGatherTiles[] = {
-    {64, 256, 64, 64, 1.00f},     {128, 128, 64, 64, 1.00f},    {64, 128, 32, 64, 0.92f},
+    {64, 256, 64, 64, 1.00f},     {128, 256, 64, 64, 2.00f, 32, 0, 1}, {64, 128, 32, 64, 0.92f},
     {32, 256, 32, 64, 0.90f},     {16, 256, 16, 64, 0.80f},     {64, 64, 32, 32, 0.80f},
     {64, 64, 32, 32, 0.90f, 64},  {64, 128, 32, 64, 0.95f, 32}, {128, 64, 64, 32, 0.95f, 32},
     {64, 64, 32, 32, 0.85f, 16, 4}, {64, 128, 32, 64, 0.95f, 16, 3}, {64, 64, 32, 32, 0.90f, 32, 3},
-    {64, 128, 32, 64, 0.97f, 32, 2}, {64, 128, 32, 64, 0.95f, 16, 0, 1},
+    {64, 128, 32, 64, 0.97f, 32, 2}, {64, 128, 32, 64, 0.95f, 16, 0, 0, 1},
     {32, 64, 16, 32, 0.60f}, {32, 64, 16, 32, 0.65f, 32}, {32, 64, 16, 32, 0.65f, 64},
-    {256, 32, 64, 32, 1.00f, 16, 0, 2}, {128, 32, 32, 32, 1.00f, 16, 0, 2}, {128, 64, 32, 64, 1.00f, 16, 0, 2},
+    {256, 32, 64, 32, 1.00f, 16, 0, 0, 2}, {128, 32, 32, 32, 1.00f, 16, 0, 0, 2}, {128, 64, 32, 64, 1.00f, 16, 0, 0, 2},
 };
 // Plan tile index t < 3 * kNGather: kGatherTiles[t % kNGather] in one of three variants. t < kNGather: tap-major K
 // order where it applies, over a re-packed filter; kNGather <= t < 2 kNGather: channel-major order (no filter
@@ -1918,20 +2282,32 @@ static const Tile& gtile(int t) { return kGatherTiles[t % kNGather]; }
 static bool gcm(int t) { return t >= kNGather && t < 2 * kNGather; }
 static bool wplace_tile(int t) {
   const Tile& tl = gtile(t);
-  return t >= 2 * kNGather && !tl.stream && tl.bp * tl.bk >= 1024;
+  return t >= 2 * kNGather && !tl.stream && !tl.split && tl.bp * tl.bk >= 1024;
+}
+// The split tile's rows: 128, or 64 where that leaves at least an eighth less padding (64 x 256 splits
+// each source value for half as many products: 64 output channels at 56x56, batch 256, take 465 us on it and 65, on
+// half-empty 128-row tiles, 576).
+static int split_bp(int64_t P) { return 8 * (cdiv(P, 64) * 64) <= 7 * (cdiv(P, 128) * 128) ? 64 : 128; }
+static int tile_bp(const Tile& tl, int64_t P) { return tl.split ? split_bp(P) : tl.bp; }
+// An upper bound on the bytes of the split tile's packed filter (z phases of at most K); past 2 GiB its plans run as
+// tile 2.
+static bool split_fits(int64_t P, int64_t K, int64_t z) { return z * (P + 128) * (K + 32) * 6 <= kMaxBufBytes; }
+// Whether the split tile is among the plans to choose from: 2^30 multiply-adds or more (z phases of P x Q x K). Below
+// that the smaller fp32 tiles fill the GPU better and its filter pack is a launch too many: 64 channels over 32 images
+// of 16 x 16 (0.3 x 2^30) take 15 us on the tuned fp32 tile and 28 on the split tile in its best K split; 256 over 64
+// images of 14 x 14 (6.9 x 2^30) 167 and 114, 64 over 64 images of 28 x 28 (1.7 x 2^30) 50 and 40.
+static bool split_pays(int64_t P, int64_t Q, int64_t K, int64_t z) {
+  return split_fits(P, K, z) && P * Q * K * z >= ((int64_t)1 << 30);
 }
 
 static const Tile kWgradTiles[] = {
     {64, 128, 32, 64, 1.00f}, {128, 64, 32, 64, 1.00f}, {64, 64, 32, 32, 0.85f}, {32, 128, 16, 64, 0.85f},
 };
 
-constexpr int64_t kCUs = 256;
-
 template <int MODE, bool BN>
 static void gather_dispatch(int ti, const GatherArgs& a, dim3 grid, hipStream_t s) {
   switch (ti) {
     case 0: hipLaunchKernelGGL((conv_gather_kernel<64, 256, 64, 64, 16, MODE, BN, BN ? 1 : 2>), grid, dim3(256), 0, s, a); break;
-    case 1: hipLaunchKernelGGL((conv_gather_kernel<128, 128, 64, 64, 16, MODE, BN, 2>), grid, dim3(256), 0, s, a); break;
     case 2: hipLaunchKernelGGL((conv_gather_kernel<64, 128, 32, 64, 16, MODE, BN, 2>), grid, dim3(256), 0, s, a); break;
     case 3: hipLaunchKernelGGL((conv_gather_kernel<32, 256, 32, 64, 16, MODE, BN, 2>), grid, dim3(256), 0, s, a); break;
     case 4: hipLaunchKernelGGL((conv_gather_kernel<16, 256, 16, 64, 16, MODE, BN, 2>), grid, dim3(256), 0, s, a); break;
@@ -1955,7 +2331,6 @@ static void gather_inplace_dispatch(int ti, const GatherArgs& a, dim3 grid, hipS
   constexpr int M = kTapInPlace;
   switch (ti) {
     case 0: hipLaunchKernelGGL((conv_gather_kernel<64, 256, 64, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
-    case 1: hipLaunchKernelGGL((conv_gather_kernel<128, 128, 64, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
     case 6: hipLaunchKernelGGL((conv_gather_kernel<64, 64, 32, 32, 64, M, false, 2>), grid, dim3(256), 0, s, a); break;
     case 8: hipLaunchKernelGGL((conv_gather_kernel<128, 64, 64, 32, 32, M, false, 2>), grid, dim3(256), 0, s, a); break;
     case 2: case 10: hipLaunchKernelGGL((conv_gather_kernel<64, 128, 32, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
@@ -1974,12 +2349,43 @@ static void gather_dl_dispatch(int ti, const GatherArgs& a, dim3 grid, hipStream
   }
 }
 
+// The split tile in its K order: tap-major, channel-major, or over a channels-last source.
+template <int MODE>
+static void gather_split_dispatch(const GatherArgs& a, dim3 grid, hipStream_t s) {
+  if (split_bp(a.P) == 64)
+    hipLaunchKernelGGL((conv_gather_split_kernel<64, 256, 32, 64, MODE>), grid, dim3(kSplitNT), 0, s, a);
+  else
+    hipLaunchKernelGGL((conv_gather_split_kernel<128, 256, 64, 64, MODE>), grid, dim3(kSplitNT), 0, s, a);
+}
+// Lays out the phases of the split tile's packed filter (a.ph and a.P set) and returns its bytes.
+static size_t split_layout(GatherArgs& a) {
+  int64_t units = 0;
+  for (int f = 0; f < a.nphase; ++f) {
+    a.ph[f].soff = (int)units;
+    a.ph[f].snkb = (int)std::max<int64_t>(1, cdiv(a.ph[f].K, kSplitBK));
+    units += cdiv(a.P, split_bp(a.P)) * a.ph[f].snkb * 12 * split_bp(a.P);
+  }
+  return (size_t)units * 16;
+}
+// Packs the filter that a's fields describe (in place, or [P][K] at a.w) into `out`, of split_layout's size.
+static int launch_split_pack(GatherArgs& a, void* out, hipStream_t s) {
+  const size_t bytes = split_layout(a);
+  const int threads = (int)(bytes / 48);
+  a.wsplit = (const uint32_t*)out;
+  a.wsplit_bytes = (uint32_t)bytes;
+  const dim3 grid((unsigned)cdiv(threads, 256));
+  if (split_bp(a.P) == 64)
+    hipLaunchKernelGGL(split_pack_kernel<64>, grid, dim3(256), 0, s, a, (uint4*)out, threads);
+  else
+    hipLaunchKernelGGL(split_pack_kernel<128>, grid, dim3(256), 0, s, a, (uint4*)out, threads);
+  return launch_check("split_pack_kernel");
+}
+
 // Channels-last gathers: the staged tiles 0 .. 8 (the tile's K-block divides the source channels).
 static void gather_nhwc_dispatch(int ti, const GatherArgs& a, dim3 grid, hipStream_t s) {
   constexpr int M = kNhwc;
   switch (ti) {
     case 0: hipLaunchKernelGGL((conv_gather_kernel<64, 256, 64, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
-    case 1: hipLaunchKernelGGL((conv_gather_kernel<128, 128, 64, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
     case 2: hipLaunchKernelGGL((conv_gather_kernel<64, 128, 32, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
     case 3: hipLaunchKernelGGL((conv_gather_kernel<32, 256, 32, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
     case 4: hipLaunchKernelGGL((conv_gather_kernel<16, 256, 16, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
@@ -1991,7 +2397,7 @@ static void gather_nhwc_dispatch(int ti, const GatherArgs& a, dim3 grid, hipStre
 }
 
 // Tap-major order needs whole K-blocks of channels (so K has no tail); the BN loader keeps the channel-major order.
-static bool gather_tap_major(int64_t c, bool bn, int bk) { return !bn && c % bk == 0; }
+static bool gather_tap_major(int64_t c, bool bn, int run) { return !bn && c % run == 0; }
 
 // Tile and K split of a gather launch: P rows, Q columns (the largest phase), K the longest reduction, z phases.
 struct GatherPlan {
@@ -2010,12 +2416,13 @@ static const int kSliceChoices[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
 // nhwc_c > 0: a channels-last gather over nhwc_c source channels, which runs the staged tiles 0 .. kNhwcTiles - 1 whose
 // K-block divides nhwc_c (a fixed plan outside them runs as tile kNhwcDefault).
 constexpr int kNhwcTiles = 9, kNhwcDefault = 5;
-static bool nhwc_tile_ok(int t, int64_t c) { return t >= 0 && t < kNhwcTiles && c % kGatherTiles[t].bk == 0; }
+static bool nhwc_tile_ok(int t, int64_t c) { return t >= 0 && t < kNhwcTiles && c % kGatherTiles[t].run() == 0; }
 static GatherPlan gather_plan(int64_t P, int64_t Q, int64_t K, int64_t z, const omt_conv_plan* fixed,
                               int64_t nhwc_c = 0) {
   const int64_t kk = K > 0 ? K : 1;
   if (fixed) {
-    const int tile = nhwc_c && !nhwc_tile_ok(fixed->tile, nhwc_c) ? kNhwcDefault : fixed->tile;
+    int tile = nhwc_c && !nhwc_tile_ok(fixed->tile, nhwc_c) ? kNhwcDefault : fixed->tile;
+    if (gtile(tile).split && !split_fits(P, kk, z)) tile = 2;
     const int64_t nkb = cdiv(kk, gtile(tile).bk);
     const int64_t kb = cdiv(nkb, std::max<int64_t>(1, std::min<int64_t>(fixed->slices, nkb)));
     return {tile, cdiv(nkb, kb), kb * gtile(tile).bk};
@@ -2026,7 +2433,9 @@ static GatherPlan gather_plan(int64_t P, int64_t Q, int64_t K, int64_t z, const 
     const Tile& tl = kGatherTiles[ti];
     if (tl.stream) continue;  // chosen by tuning only
     if (nhwc_c && !nhwc_tile_ok(ti, nhwc_c)) continue;
-    const int64_t tiles = cdiv(P, tl.bp) * cdiv(Q, tl.bq) * z, nkb = cdiv(kk, tl.bk);
+    if (tl.split && !split_pays(P, Q, kk, z)) continue;
+    const int bp = tile_bp(tl, P);
+    const int64_t tiles = cdiv(P, bp) * cdiv(Q, tl.bq) * z, nkb = cdiv(kk, tl.bk);
     for (int sc : kSliceChoices) {
       const int64_t kb = cdiv(nkb, sc);
       if (sc > 1 && kb * tl.bk < 96) break;
@@ -2034,9 +2443,11 @@ static GatherPlan gather_plan(int64_t P, int64_t Q, int64_t K, int64_t z, const 
       if (slices != sc) continue;
       const int64_t blocks = tiles * slices;
       const bool alone = blocks <= kCUs;
-      const double blk = std::max((double)tl.bp * tl.bq * tl.bk / (34.0 * tl.eff) / (alone ? 1.6 : 1.0),
+      // the split tile runs one workgroup of eight waves per CU
+      const double wgs = tl.split ? 1.0 : 2.0;
+      const double blk = std::max((double)bp * tl.bq * tl.bk * wgs / (68.0 * tl.eff) / (alone && !tl.split ? 1.6 : 1.0),
                                   alone ? 2000.0 : 1000.0);
-      double cost = blk * (kb + 2) * (alone ? 1.0 : (double)cdiv(blocks, 2 * kCUs));
+      double cost = blk * (kb + 2) * (alone ? 1.0 : (double)cdiv(blocks, (int64_t)wgs * kCUs));
       if (slices > 1) cost += 7000.0 + (double)(2 * slices) * P * Q * z * 4 / 1700.0;
       if (cost < best_cost * 0.999) {
         best_cost = cost;
@@ -2076,7 +2487,7 @@ static dim3 gather_grid(GatherArgs& a, const GatherPlan& pl, int64_t n, int64_t 
     a.tpw = (int)std::max<int64_t>(1, cdiv(ntq * ntp, (a.stats ? 3 : 4) * kCUs));
     return dim3((unsigned)cdiv(ntq, a.tpw), (unsigned)ntp, 1);
   }
-  return dim3((unsigned)cdiv(maxq, tl.bq), (unsigned)cdiv(a.P, tl.bp), (unsigned)(a.nphase * pl.slices));
+  return dim3((unsigned)cdiv(maxq, tl.bq), (unsigned)cdiv(a.P, tile_bp(tl, a.P)), (unsigned)(a.nphase * pl.slices));
 }
 // The 1x1 streaming tile runs only where its kernel applies (one 1x1 stride-1 unpadded phase, the [P][K] filter in
 // place or re-packed, no BN loader, no split K, whole K-blocks, float4 runs of output pixels inside one image and
@@ -2093,14 +2504,16 @@ static bool wst_ok(const GatherArgs& a, const GatherPlan& pl) {
   return stream_ok(a, pl) && (K == 64 || K == 128) && !a.stats && (uintptr_t)a.x % 16 == 0 &&
          (int64_t)a.ph[0].Q * a.P * 4 <= kMaxBufBytes;
 }
+// The split tile has no BN loader: its plans run as tile 2 there.
 static GatherPlan eff_plan(const GatherArgs& a, GatherPlan pl) {
+  if (gtile(pl.tile).split && a.bn_mean) pl.tile = pl.tile - pl.tile % kNGather + 2;
   if (gtile(pl.tile).stream == 2 && !wst_ok(a, pl)) pl.tile = pl.tile - pl.tile % kNGather + kStreamTile;
   if (gtile(pl.tile).stream && !stream_ok(a, pl)) pl.tile = pl.tile - pl.tile % kNGather + 2;
   return pl;
 }
 // Tap-major K order of a gather launch (the BN loader keeps the channel-major order).
 static bool gather_uses_tap_major(const GatherArgs& a, const GatherPlan& pl) {
-  return !a.bn_mean && !gcm(pl.tile) && gather_tap_major(a.C, false, gtile(pl.tile).bk);
+  return !a.bn_mean && !gcm(pl.tile) && gather_tap_major(a.C, false, gtile(pl.tile).run());
 }
 // The slice sum of a split gather launch (blocks 0 if the plan does not split).
 static GatherSum gather_sum_of(const GatherArgs& a, const GatherPlan& pl) {
@@ -2170,7 +2583,11 @@ static int run_gather(GatherArgs& a, const GatherPlan& plan, int64_t n, int64_t 
       hipLaunchKernelGGL((conv1x1_stream_kernel<64, 128, 32, 64, false>), grid, dim3(256), 0, s, a, a.tpw);
     return launch_check("conv1x1_stream_kernel");
   }
-  if (a.bn_mean)
+  if (gtile(pl.tile).split && gather_uses_tap_major(a, pl))
+    gather_split_dispatch<kTapMajor>(a, grid, s);
+  else if (gtile(pl.tile).split)
+    gather_split_dispatch<kGeneric>(a, grid, s);
+  else if (a.bn_mean)
     gather_dispatch<kGeneric, true>(pl.tile % kNGather, a, grid, s);
   else if (a.wplace)
     gather_inplace_dispatch(pl.tile % kNGather, a, grid, s);
@@ -2337,10 +2754,17 @@ static GatherPlan fwd_plan(const omt_conv_geo* g) {
   const bool have = cached_plan(OMT_DIR_FWD, g, &cp);
   return gather_plan(g->co, g->n * g->oh * g->ow, g->ci * g->ks * g->ks, 1, have ? &cp : nullptr);
 }
-// Forward workspace: the tap-major filter (when the plan's K-block divides C and ks > 1), then, 256-byte aligned,
-// the split-K partials.
+// Forward workspace: the tap-major filter (when the plan's K-block divides C and ks > 1), or the split tile's packed
+// filter, then, 256-byte aligned, the split-K partials.
 static size_t fwd_pack_bytes(const omt_conv_geo* g, const GatherPlan& pl) {
-  if (g->ks == 1 || gcm(pl.tile) || wplace_tile(pl.tile) || !gather_tap_major(g->ci, false, gtile(pl.tile).bk))
+  if (gtile(pl.tile).split) {
+    GatherArgs a{};
+    a.P = (int)g->co;
+    a.nphase = 1;
+    a.ph[0].K = (int)(g->ci * g->ks * g->ks);
+    return split_layout(a);
+  }
+  if (g->ks == 1 || gcm(pl.tile) || wplace_tile(pl.tile) || !gather_tap_major(g->ci, false, gtile(pl.tile).run()))
     return 0;
   return (size_t)(g->co * g->ci * g->ks * g->ks) * sizeof(float);
 }
@@ -2376,18 +2800,21 @@ static int conv_fwd_one(const omt_conv_geo* g, const float* x, const float* w, c
   a.x = x;
   a.w = w;
   // tap-major order: re-pack the filter to [co][ky][kx][ci] (1x1 filters already are)
-  if (!bn && fwd_pack_bytes(g, pl)) {
+  const bool split = !bn && gtile(pl.tile).split;
+  if (!bn && !split && fwd_pack_bytes(g, pl)) {
     const int total = (int)(g->co * g->ci * g->ks * g->ks);
     hipLaunchKernelGGL(pack_tapmajor_kernel, dim3(grid1d(total, 256, 4096)), dim3(256), 0, s, w, (float*)workspace,
                        (int)g->co, (int)g->ci, (int)(g->ks * g->ks));
     if (int st = launch_check("pack_tapmajor_kernel")) return st;
     a.w = (const float*)workspace;
   }
-  if (!bn && g->ks > 1 && wplace_tile(pl.tile) && gather_tap_major(g->ci, false, gtile(pl.tile).bk)) {
+  if (!bn && (split ? !gcm(pl.tile) : g->ks > 1 && wplace_tile(pl.tile)) &&
+      gather_tap_major(g->ci, false, gtile(pl.tile).run())) {
     a.wplace = 1;  // A[co][(ky, kx, ci)] = w[co][ci][ky][kx]
     a.ks = (int)g->ks;
     a.w_rowst = (uint32_t)(g->ci * g->ks * g->ks * 4);
     a.w_cst = (uint32_t)(g->ks * g->ks * 4);
+    a.w_tst = 4;
   }
   a.bias = (epilogue & OMT_EPI_BIAS) ? bias : nullptr;
   a.bn_mean = bn ? bn_mean : nullptr;
@@ -2422,6 +2849,8 @@ static int conv_fwd_one(const omt_conv_geo* g, const float* x, const float* w, c
   p.div_kk = make_fastdiv((uint32_t)(g->ks * g->ks));
   p.div_kw = make_fastdiv((uint32_t)g->ks);
   a.div_c = make_fastdiv((uint32_t)a.C);
+  if (split)
+    if (int st = launch_split_pack(a, workspace, s)) return st;
   float* part = (float*)((char*)workspace + align256(fwd_pack_bytes(g, pl)));
   if (parts) *parts = part;
   if (stats) {  // the statistics come from the epilogue of an unsplit plan (checked above, before any launch)
@@ -2596,13 +3025,26 @@ static GatherPlan dgrad_plan(const omt_conv_geo* g) {
 
 // Grad input re-packs its filter for the tap-major order only (the channel-major order reads w directly), and always
 // in the super-pixel form.
+static size_t d2s_pack_bytes(const omt_conv_geo* g) {
+  int L = 1, PH = 0;
+  d2s_window(g, L, PH);
+  return (size_t)(g->stride * g->stride * g->ci * g->co * L * L) * sizeof(float);
+}
 static size_t dgrad_pack_bytes(const omt_conv_geo* g, const GatherPlan& pl) {
-  if (dgrad_d2s(g)) {
-    int L = 1, PH = 0;
-    d2s_window(g, L, PH);
-    return (size_t)(g->stride * g->stride * g->ci * g->co * L * L) * sizeof(float);
+  if (gtile(pl.tile).split) {  // the split tile's packed filter, after the super-pixel filter it is packed from
+    GatherArgs a{};
+    PackArgs pk{};
+    int64_t maxq = 0;
+    const bool d2s = dgrad_d2s(g);
+    if (d2s)
+      dgrad_d2s_phase(g, a, maxq);
+    else
+      dgrad_phases(g, a, pk, maxq);
+    a.P = (int)(d2s ? g->stride * g->stride * g->ci : g->ci);
+    return (d2s ? align256(d2s_pack_bytes(g)) : 0) + split_layout(a);
   }
-  if (gcm(pl.tile) || wplace_tile(pl.tile) || !gather_tap_major(g->co, false, gtile(pl.tile).bk)) return 0;
+  if (dgrad_d2s(g)) return d2s_pack_bytes(g);
+  if (gcm(pl.tile) || wplace_tile(pl.tile) || !gather_tap_major(g->co, false, gtile(pl.tile).run())) return 0;
   return (size_t)(g->co * g->ci * g->ks * g->ks) * sizeof(float);
 }
 
@@ -2643,6 +3085,7 @@ static int dgrad_prepare(const omt_conv_geo* g, const float* gy, const float* w,
   const int packed = d2s ? 0 : dgrad_phases(g, a, pk, maxq);
   pl = dgrad_plan(g);
   const size_t pack = dgrad_pack_bytes(g, pl);
+  const bool split = gtile(pl.tile).split;
   if (d2s) {
     dgrad_d2s_phase(g, a, maxq);
     PackD2S pd{};
@@ -2655,15 +3098,22 @@ static int dgrad_prepare(const omt_conv_geo* g, const float* gy, const float* w,
     pd.PAD = (int)g->pad;
     pd.L = a.ph[0].KH;
     pd.PH = a.ph[0].PH;
-    pd.tap_major = !gcm(pl.tile) && gather_tap_major(g->co, false, gtile(pl.tile).bk);
-    const int64_t total = (int64_t)(pack / sizeof(float));
+    pd.tap_major = !gcm(pl.tile) && gather_tap_major(g->co, false, gtile(pl.tile).run());
+    const int64_t total = (int64_t)(d2s_pack_bytes(g) / sizeof(float));
     hipLaunchKernelGGL(pack_d2s_weights_kernel, dim3(grid1d(total, 256, 4096)), dim3(256), 0, s, pd);
     if (int st = launch_check("pack_d2s_weights_kernel")) return st;
     a.w = (const float*)workspace;
-    a.w_bytes = (uint32_t)pack;
+    a.w_bytes = (uint32_t)d2s_pack_bytes(g);
+    if (split && pd.tap_major) {  // the split tile reads the packed rows as a filter in place
+      a.wplace = 1;
+      a.ks = pd.L;
+      a.w_rowst = (uint32_t)(a.ph[0].K * 4);
+      a.w_cst = 4;
+      a.w_tst = (uint32_t)(g->co * 4);
+    }
     a.d2s = (int)g->stride;
     a.d2s_ci = (int)g->ci;
-  } else if (pack) {
+  } else if (pack && !split) {
     pk.w = w;
     pk.out = (float*)workspace;
     pk.CO = (int)g->co;
@@ -2680,10 +3130,11 @@ static int dgrad_prepare(const omt_conv_geo* g, const float* gy, const float* w,
     a.w_bytes = (uint32_t)(g->co * g->ci * g->ks * g->ks * 4);
     a.ks = (int)g->ks;
     a.s = (int)g->stride;
-    if (wplace_tile(pl.tile) && gather_tap_major(g->co, false, gtile(pl.tile).bk)) {
+    if ((split ? !gcm(pl.tile) : wplace_tile(pl.tile)) && gather_tap_major(g->co, false, gtile(pl.tile).run())) {
       a.wplace = 2;  // A[ci][(a', b', co)] = w[co][ci][ky0 + s (KH - 1 - a')][kx0 + s (KW - 1 - b')]
       a.w_rowst = (uint32_t)(g->ks * g->ks * 4);
       a.w_cst = (uint32_t)(g->ci * g->ks * g->ks * 4);
+      a.w_tst = 4;
     } else {
       a.wdirect = 1;
     }
@@ -2701,6 +3152,7 @@ static int dgrad_prepare(const omt_conv_geo* g, const float* gy, const float* w,
   a.d2s_w = (int)g->iw;
   a.div_c = make_fastdiv((uint32_t)a.C);
   part = workspace ? (float*)((char*)workspace + align256(pack)) : nullptr;
+  if (split) return launch_split_pack(a, (char*)workspace + (d2s ? align256(d2s_pack_bytes(g)) : 0), s);
   return OMT_OK;
 }
 
@@ -3136,8 +3588,10 @@ static int run_gather_nhwc(GatherArgs& a, const GatherPlan& pl, int64_t n, int64
   a.tpw = 0;
   a.rows = 0;
   a.vec_out = a.P % 4 == 0 && (uintptr_t)a.y % 16 == 0 && (uintptr_t)a.part % 16 == 0;
-  const dim3 grid((unsigned)cdiv(maxq, tl.bq), (unsigned)cdiv(a.P, tl.bp), (unsigned)(a.nphase * pl.slices));
-  if (narrow)
+  const dim3 grid((unsigned)cdiv(maxq, tl.bq), (unsigned)cdiv(a.P, tile_bp(tl, a.P)), (unsigned)(a.nphase * pl.slices));
+  if (tl.split)
+    gather_split_dispatch<kNhwc>(a, grid, s);
+  else if (narrow)
     hipLaunchKernelGGL((conv_gather_kernel<64, 64, 32, 32, 16, kNhwcNarrow, false, 2>), grid, dim3(256), 0, s, a);
   else
     gather_nhwc_dispatch(pl.tile, a, grid, s);
@@ -3145,10 +3599,15 @@ static int run_gather_nhwc(GatherArgs& a, const GatherPlan& pl, int64_t n, int64
   return launch_gather_sum(gather_sum_of(a, pl), s);
 }
 
+// The split tile's packed filter, then, 256-byte aligned, any split-K partials.
+static size_t fwd_nhwc_pack_bytes(const omt_conv_geo* g, const GatherPlan& pl) {
+  return gtile(pl.tile).split ? fwd_pack_bytes(g, pl) : 0;
+}
 static size_t fwd_nhwc_workspace_one(const omt_conv_geo* g) {
   if (nhwc_narrow(g)) return 0;
   const GatherPlan pl = fwd_nhwc_plan(g);
-  return pl.slices > 1 ? (size_t)(pl.slices * g->n * g->co * g->oh * g->ow) * sizeof(float) : 0;
+  const size_t pack = fwd_nhwc_pack_bytes(g, pl);
+  return pl.slices > 1 ? align256(pack) + (size_t)(pl.slices * g->n * g->co * g->oh * g->ow) * sizeof(float) : pack;
 }
 
 OMT_EXPORT size_t omt_conv_fwd_nhwc_workspace(const omt_conv_geo* g) {
@@ -3189,7 +3648,10 @@ static int conv_fwd_nhwc_one(const omt_conv_geo* g, const float* x, const float*
   p.div_kk = make_fastdiv((uint32_t)(g->ks * g->ks));
   p.div_kw = make_fastdiv((uint32_t)g->ks);
   a.div_c = make_fastdiv((uint32_t)a.C);
-  return run_gather_nhwc(a, pl, g->n, p.Q, (float*)workspace, s, narrow);
+  if (gtile(pl.tile).split)
+    if (int st = launch_split_pack(a, workspace, s)) return st;
+  float* part = (float*)((char*)workspace + align256(narrow ? 0 : fwd_nhwc_pack_bytes(g, pl)));
+  return run_gather_nhwc(a, pl, g->n, p.Q, part, s, narrow);
 }
 
 OMT_EXPORT int omt_conv_fwd_nhwc(const omt_conv_geo* g, const float* x, const float* w, const float* bias,
@@ -3209,10 +3671,20 @@ OMT_EXPORT int omt_conv_fwd_nhwc(const omt_conv_geo* g, const float* x, const fl
 }
 
 // Grad-input workspace: the per-phase filters W'[ci][a'][b'][co] (all of the filter's elements), then, 256-byte
-// aligned, any split-K partials [slices][n][ih][iw][ci].
+// aligned each, the split tile's packed filter and any split-K partials [slices][n][ih][iw][ci].
+static size_t dgrad_nhwc_pack_bytes(const omt_conv_geo* g, const GatherPlan& pl) {
+  const size_t pack = (size_t)(g->co * g->ci * g->ks * g->ks) * sizeof(float);
+  if (!gtile(pl.tile).split) return pack;
+  GatherArgs a{};
+  PackArgs pk{};
+  int64_t maxq = 0;
+  dgrad_phases(g, a, pk, maxq);
+  a.P = (int)g->ci;
+  return align256(pack) + split_layout(a);
+}
 static size_t dgrad_nhwc_workspace_one(const omt_conv_geo* g) {
   const GatherPlan pl = dgrad_nhwc_plan(g);
-  const size_t pack = (size_t)(g->co * g->ci * g->ks * g->ks) * sizeof(float);
+  const size_t pack = dgrad_nhwc_pack_bytes(g, pl);
   return pl.slices > 1 ? align256(pack) + (size_t)(pl.slices * g->n * g->ci * g->ih * g->iw) * sizeof(float) : pack;
 }
 
@@ -3257,7 +3729,9 @@ static int conv_dgrad_nhwc_one(const omt_conv_geo* g, const float* gy, const flo
   a.YH = (int)g->ih;
   a.YW = (int)g->iw;
   a.div_c = make_fastdiv((uint32_t)a.C);
-  float* part = (float*)((char*)workspace + align256((size_t)packed * sizeof(float)));
+  if (gtile(pl.tile).split)
+    if (int st = launch_split_pack(a, (char*)workspace + align256((size_t)packed * sizeof(float)), s)) return st;
+  float* part = (float*)((char*)workspace + align256(dgrad_nhwc_pack_bytes(g, pl)));
   return run_gather_nhwc(a, pl, g->n, maxq, part, s, nhwc_dgrad_narrow(g));
 }
 
@@ -3460,12 +3934,13 @@ std::vector<omt_conv_plan> tune_candidates(int dir, const omt_conv_geo* g, int n
   for (int t = 0; t < ntile; ++t) {
     const Tile& tl = gtile(t);
     if (nhwc && !nhwc_tile_ok(t, gather_c)) continue;
-    if (t >= 2 * kNGather && !(wplace_tile(t) && packs && gather_tap_major(gather_c, false, tl.bk))) continue;
+    if (tl.split && (t >= kNGather || !split_pays(P, Q, K, z))) continue;  // its variants differ in K order alone
+    if (t >= 2 * kNGather && !(wplace_tile(t) && packs && gather_tap_major(gather_c, false, tl.run()))) continue;
     if (tl.stream) {
       if (stream_geo && t < kNGather && (tl.stream == 1 || K == 64 || K == 128)) out.push_back({t, 1});
       continue;
     }
-    const int64_t tiles = cdiv(P, tl.bp) * cdiv(Q, tl.bq) * z, nkb = cdiv(std::max<int64_t>(K, 1), tl.bk);
+    const int64_t tiles = cdiv(P, tile_bp(tl, P)) * cdiv(Q, tl.bq) * z, nkb = cdiv(std::max<int64_t>(K, 1), tl.bk);
     // A grid that already fills the GPU is split only to even out its last round: a few workgroups per CU, all
     // resident at once, finish when the CUs holding one more than the rest do (1568 tiles: 7 on some CUs, 6.125 on
     // average); 2-4 slices of at least 8 K-blocks each spread them more evenly.
@@ -3484,6 +3959,9 @@ std::vector<omt_conv_plan> tune_candidates(int dir, const omt_conv_geo* g, int n
   return out;
 }
 
+// Whether a plan runs a split tile.
+bool split_plan(int dir, const omt_conv_plan& p) { return !wgrad_dir(dir) && gtile(p.tile).split; }
+
 bool forcing() {
   for (const auto* f : t_force)
     if (f) return true;
@@ -3496,8 +3974,20 @@ struct ForceGuard {
   }
 };
 
-// Scratch buffers, events and a private stream of one tuning run: zero inputs (fp32 MFMA timing does not depend on
-// the values). Candidates are timed as replays of a captured HIP graph on the private stream, the way a training step
+// Values of both signs and many exponents for the tuner's scratch inputs where a split tile is among the candidates:
+// the matrix cores draw less power on zeros and clock higher (bf16 2411 TFLOP/s on zeros, 1988 on random values; fp32
+// 156 and 146), which would favour them.
+__global__ void __launch_bounds__(256) tune_fill_kernel(float* p, int64_t n) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    uint32_t h = (uint32_t)i * 2654435761u;
+    h ^= h >> 15;
+    h *= 2246822519u;
+    h ^= h >> 13;
+    p[i] = (float)(int32_t)h * (1.f / 2147483648.f);
+  }
+}
+
+// Scratch buffers, events and a private stream of one tuning run: zero inputs, or random ones (above). Candidates are timed as replays of a captured HIP graph on the private stream, the way a training step
 // runs: each extra launch of a plan (filter re-pack, split-K slice sum) then costs what a graph node costs, which
 // back-to-back stream launches hide. The destructor synchronizes both streams, so nothing queued still uses the buffers
 // when they return to the cache.
@@ -3506,7 +3996,7 @@ struct TuneScratch {
   void *x = nullptr, *w = nullptr, *gy = nullptr, *o1 = nullptr, *o2 = nullptr, *ws = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   explicit TuneScratch(hipStream_t st) : s(st) {}
-  int init(const omt_conv_geo* g, size_t ws_bytes) {
+  int init(const omt_conv_geo* g, size_t ws_bytes, bool random) {
     const size_t xb = (size_t)(g->n * g->ci * g->ih * g->iw) * 4, wb = (size_t)(g->co * g->ci * g->ks * g->ks) * 4,
                  yb = (size_t)(g->n * g->co * g->oh * g->ow) * 4;
     const size_t ob = std::max(xb, std::max(wb, yb));
@@ -3517,13 +4007,19 @@ struct TuneScratch {
     if (int st = omt_malloc_on(&o2, wb, s)) return st;
     if (ws_bytes)
       if (int st = omt_malloc_on(&ws, ws_bytes, s)) return st;
-    if (int st = hip_check(hipMemsetAsync(x, 0, xb, s), "hipMemsetAsync")) return st;
-    if (int st = hip_check(hipMemsetAsync(w, 0, wb, s), "hipMemsetAsync")) return st;
-    if (int st = hip_check(hipMemsetAsync(gy, 0, yb, s), "hipMemsetAsync")) return st;
+    for (auto [p, b] : {std::pair<void*, size_t>{x, xb}, {w, wb}, {gy, yb}}) {
+      if (!random) {
+        if (int st = hip_check(hipMemsetAsync(p, 0, b, s), "hipMemsetAsync")) return st;
+        continue;
+      }
+      const int64_t n = (int64_t)(b / 4);
+      hipLaunchKernelGGL(tune_fill_kernel, dim3(grid1d(n, 256, 8192)), dim3(256), 0, s, (float*)p, n);
+      if (int st = launch_check("tune_fill_kernel")) return st;
+    }
     if (int st = hip_check(hipEventCreate(&e0), "hipEventCreate")) return st;
     if (int st = hip_check(hipEventCreate(&e1), "hipEventCreate")) return st;
     if (int st = hip_check(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking), "hipStreamCreateWithFlags")) return st;
-    // the private stream starts after the zeroing queued on s
+    // the private stream starts after the fills queued on s
     if (int st = hip_check(hipEventRecord(e0, s), "hipEventRecord")) return st;
     return hip_check(hipStreamWaitEvent(cs, e0, 0), "hipStreamWaitEvent");
   }
@@ -3603,6 +4099,7 @@ OMT_EXPORT int omt_conv_autotune(int dir, const omt_conv_geo* g, int max_tiles, 
   const std::vector<omt_conv_plan> cands = tune_candidates(dir, g, ntile);
   if (cands.empty()) return fail(OMT_UNSUPPORTED, "omt_conv_autotune: no candidate plan");
 
+  const bool random = std::any_of(cands.begin(), cands.end(), [&](const omt_conv_plan& c) { return split_plan(dir, c); });
   ForceGuard guard;
   size_t ws_bytes = 0;
   for (const omt_conv_plan& c : cands) {
@@ -3613,7 +4110,7 @@ OMT_EXPORT int omt_conv_autotune(int dir, const omt_conv_geo* g, int max_tiles, 
   omt_conv_plan win = cands[0];
   {
     TuneScratch sc(s);
-    if (int st = sc.init(g, ws_bytes)) return st;
+    if (int st = sc.init(g, ws_bytes, random)) return st;
     auto run = [&](hipStream_t rs) -> int {
       const size_t need = dir_workspace(dir, g);
       const float *x = (const float*)sc.x, *w = (const float*)sc.w, *gy = (const float*)sc.gy;
@@ -3675,6 +4172,7 @@ OMT_EXPORT int omt_conv_autotune_bwd(const omt_conv_geo* g, int max_tiles, void*
     for (const omt_conv_plan& d : ds)
       for (const omt_conv_plan& w : wsv) cands.push_back({d, w});
   }
+  const bool random = split_plan(OMT_DIR_DGRAD, dsep) || split_plan(OMT_DIR_WGRAD, wsep);
   ForceGuard guard;
   size_t ws_bytes = 0;
   for (const auto& c : cands) {
@@ -3686,7 +4184,7 @@ OMT_EXPORT int omt_conv_autotune_bwd(const omt_conv_geo* g, int max_tiles, void*
   std::pair<omt_conv_plan, omt_conv_plan> win = cands[0];
   {
     TuneScratch sc(s);
-    if (int st = sc.init(g, ws_bytes)) return st;
+    if (int st = sc.init(g, ws_bytes, random)) return st;
     auto run = [&](hipStream_t rs) -> int {
       return omt_conv_bwd(g, (const float*)sc.x, (const float*)sc.gy, (const float*)sc.w, (float*)sc.o1,
                           (float*)sc.o2, sc.ws, omt_conv_bwd_workspace(g), rs);

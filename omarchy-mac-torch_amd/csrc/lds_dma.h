@@ -32,6 +32,13 @@ __device__ __forceinline__ void lds_load_b32(omt_u32x4 r, uint32_t m0, uint32_t 
                : "s"(m0), "v"(voff), "s"(r), "s"(soff)
                : "memory", "m0");
 }
+// lane i's 16 bytes at voff + soff land at LDS byte address m0 + 16 i
+__device__ __forceinline__ void lds_load_b128s(omt_u32x4 r, uint32_t m0, uint32_t voff, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "s"(m0), "v"(voff), "s"(r), "s"(soff)
+               : "memory", "m0");
+}
 // lane i's 16 bytes at voff land at LDS byte address m0 + 16 i
 __device__ __forceinline__ void lds_load_b128(omt_u32x4 r, uint32_t m0, uint32_t voff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"

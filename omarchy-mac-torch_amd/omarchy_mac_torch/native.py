@@ -197,11 +197,12 @@ FALLBACKS = _FallbackView()
 
 # ---- on-disk conv plan cache (reference: omarchy_mac_torch/native.py:185-209) ----
 # One JSON object {"dir,n,ci,co,ih,iw,oh,ow,ks,stride,pad": [tile, slices]}, the reference's key format. The values
-# index this library's gfx950 tile tables (the file name carries the gather table's size), so the file is not the
-# reference's, whose entries name its own tiles and a split-K multiplier.
+# index this library's gfx950 tile tables (the file name carries the gather table's size and its revision, so that
+# plans chosen among another table's kernels are not read), so the file is not the reference's, whose entries name its
+# own tiles and a split-K multiplier.
 TUNE_FILE = os.environ.get(
     "OMARCHY_MAC_TORCH_TUNE_FILE",
-    os.path.expanduser(f"~/.cache/omarchy-mac-torch/tuning-gfx950-t{_lib.L.omt_conv_num_tiles(_lib.OMT_DIR_FWD) // 3}.json"))
+    os.path.expanduser(f"~/.cache/omarchy-mac-torch/tuning-gfx950-t{_lib.L.omt_conv_num_tiles(_lib.OMT_DIR_FWD) // 3}r2.json"))
 
 
 class TuningStore:

@@ -1,0 +1,99 @@
+"""The split-bf16 convolution tiles (fp32 products as six bf16 products): every edge of the tile against the float64
+oracle with no more error than the fp32 tile of the same layer, and the inputs that a bf16 split cannot carry."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from oracle import oracle as orc  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+SPLIT, FP32 = 1, 2  # gather tiles
+_CL = torch.channels_last
+
+
+@pytest.fixture(scope="module")
+def ops(cuda):
+    from omarchy_mac_torch import hip_ops
+    return hip_ops
+
+
+def rnd(rng, *shape, scale=1.0):
+    return (rng.standard_normal(shape) * scale).astype(np.float32)
+
+
+def run(ops, d, t, x, w, gy, s, p, tile, slices=1):
+    ops.set_conv_plan(d, x.shape, w.shape, s, p, tile, slices)
+    y = {"fwd": lambda: ops.conv2d(t[0], t[1], None, s, p), "fwd_nhwc": lambda: ops.conv2d_nhwc(t[0], t[1], None, s, p),
+         "dgrad": lambda: ops.conv2d_dgrad(t[2], t[1], x.shape, s, p),
+         "dgrad_nhwc": lambda: ops.conv2d_dgrad_nhwc(t[2], t[1], x.shape, s, p)}[d]()
+    return y.contiguous().cpu().numpy()
+
+
+# n, ci, co, h, w, ks, stride, pad: output rows around 64 and 128 (both tile heights), pixels around 256, reductions
+# with an odd half K-block (C of 16 and 48 with 9 taps), runs that cross two taps (C of 16), any channels
+SHAPES = [
+    (1, 16, 64, 15, 17, 3, 1, 1), (1, 48, 65, 16, 16, 3, 1, 1), (2, 32, 128, 11, 12, 1, 1, 0),
+    (1, 64, 129, 257, 1, 1, 1, 0), (3, 33, 63, 9, 11, 3, 1, 1), (2, 7, 200, 10, 13, 5, 2, 2),
+    (2, 80, 48, 12, 9, 3, 2, 1), (2, 128, 16, 7, 7, 3, 1, 1), (1, 3, 64, 33, 29, 7, 2, 3), (40, 17, 31, 1, 1, 1, 1, 0),
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_split_tile_is_as_exact_as_the_fp32_tile(cuda, ops, shape):
+    """Forward and grad input, both memory formats, 1 and 3 K slices. The float64 oracle is the reference: the split
+    tile may be off by as much as the fp32 tile is, or by one rounding of the result (2^-24 each, relative)."""
+    n, ci, co, h, w, ks, s, p = shape
+    rng = np.random.default_rng(sum(shape))
+    x, wt = rnd(rng, n, ci, h, w), rnd(rng, co, ci, ks, ks, scale=(ci * ks * ks) ** -0.5)
+    y = orc.conv_fwd(x, wt, None, s, p)
+    gy = rnd(rng, *y.shape)
+    gx = orc.conv_dgrad(gy, wt, x.shape, s, p)
+    try:
+        for d, ref in (("fwd", y), ("dgrad", gx), ("fwd_nhwc", y), ("dgrad_nhwc", gx)):
+            t = [torch.from_numpy(a).to(cuda) for a in (x, wt, gy)]
+            t = [a.contiguous(memory_format=_CL) for a in t] if d.endswith("nhwc") else t
+            for slices in (1, 3):
+                e32 = orc.rel_l2(run(ops, d, t, x, wt, gy, s, p, FP32, slices), ref)
+                err = orc.rel_l2(run(ops, d, t, x, wt, gy, s, p, SPLIT, slices), ref)
+                assert err <= max(e32, 2.0 ** -24), (d, slices, err, e32)
+    finally:
+        ops.clear_conv_plans()
+
+
+@pytest.mark.parametrize("kind", ["inf", "nan", "huge", "tiny", "overflow"])
+def test_split_tile_falls_back_on_values_it_cannot_split(cuda, ops, kind):
+    """Infinities, NaN, values that round past the largest bf16, sums that overflow, and inputs whose low terms
+    underflow: the tile is computed again in fp32, so every output is the fp32 tile's to the bit where the whole tile
+    is affected, and equal in kind (NaN, infinity, finite within rounding) elsewhere."""
+    rng = np.random.default_rng(3)
+    n, ci, co, h = 2, 48, 96, 13
+    x, wt = rnd(rng, n, ci, h, h), rnd(rng, co, ci, 3, 3, scale=0.05)
+    if kind in ("inf", "nan"):
+        x[1, 5, 6, 7] = np.inf if kind == "inf" else np.nan
+        x[0, 9, 0, 0] = -np.inf if kind == "inf" else np.nan
+    elif kind == "huge":
+        x[1, 5, 6, 7] = np.float32(3.4e38)
+        wt *= np.float32(1e-3)
+    elif kind == "overflow":
+        x *= np.float32(1e30)
+        wt *= np.float32(1e9)
+    else:
+        x *= np.float32(2.0 ** -112)
+    t = [torch.from_numpy(a).to(cuda) for a in (x, wt)]
+    tc = [a.contiguous(memory_format=_CL) for a in t]
+    try:
+        for d, u in (("fwd", t), ("fwd_nhwc", tc)):
+            a = run(ops, d, u, x, wt, None, 1, 1, SPLIT)
+            b = run(ops, d, u, x, wt, None, 1, 1, FP32)
+            assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b))
+            assert np.array_equal(a[np.isinf(a)], b[np.isinf(b)])
+            f = np.isfinite(a)
+            if kind in ("tiny", "overflow"):
+                assert np.array_equal(a[f], b[f])
+            else:
+                scale = np.abs(b[f]).max() if kind == "huge" else np.sqrt((b[f].astype(np.float64) ** 2).mean())
+                # both within K 2^-24 relative of the exact sums (K = 432 products)
+                assert np.abs(a[f].astype(np.float64) - b[f]).max() <= 2 * 432 * 2.0 ** -24 * scale
+    finally:
+        ops.clear_conv_plans()

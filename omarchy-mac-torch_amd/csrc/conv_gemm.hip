@@ -1984,6 +1984,335 @@ __global__ void __launch_bounds__(256, 2) conv_wgrad_nhwc_kernel(const WgradArgs
   wgrad_nhwc_tile<BP, BQ, WP, WQ, PF, NARROW>(a, t.x, t.y, t.z, lds);
 }
 
+// ---- split-bf16 grad weight ---------------------------------------------------------------------------------------
+// The grad-weight GEMM with both operands split into three bf16 terms as in conv_gather_split_kernel (the same six
+// partial products, the same sums per 32 products, the same fp32 tile for what the split cannot carry). The reduction
+// runs over pixels, while a thread loads eight channels of one pixel: it stages them as one 16-byte unit of eight rows
+// (gy channels or tap columns) of one k, and the MFMA operands, which need eight k of one row, come back through the
+// transposing LDS read (ds_read_b64_tr_b16: a group of 16 lanes reads four k of 16 rows and hands lane r row r's four).
+// Unit (term z, rows 8 c .. 8 c + 7, k) lies at (z R / 8 + c) 32 + (k ^ 4 (c & 1)): the 4 k of two neighbouring c that
+// a group reads, and the groups of a half wave, then touch every bank once, and a wave writes 32 contiguous units.
+// 1x1 stride-1 unpadded layers whose planes are a multiple of 4 (kPix4) load eight pixels of one channel as two 16-byte
+// loads instead, into the gather tile's layout (units of eight k of one row).
+// Columns. Where C is a multiple of 32 the tap-major tiles take the columns as q = (c / 32, tap, c % 32): the taps of
+// 32 channels, which read the same cache lines of x shifted by a pixel or a row, then follow each other in one tile and
+// find them in the L1 (256 channels at 14 x 14, batch 256, 14 slices: 432 us in the order (tap, c), 340 so). Channels
+// last a pixel's channels are whole lines in any order (300 us in the order (tap, c), 354 in the other).
+template <int BP, int BQ, int MODE>
+constexpr int wgrad_split_units() {  // of one buffer
+  return MODE == kPix4 ? 12 * (BP + 4 + BQ + 4) : 3 * (BP + BQ) / 8 * kSplitBK;
+}
+
+template <int BP, int BQ, int WP, int MODE>
+__device__ __forceinline__ void wgrad_split_tile(const WgradArgs& a, const int bx, const int by, const int bz,
+                                                 uint4* __restrict__ lds) {
+  constexpr int NT = kSplitNT, NW = NT / 64, BK = kSplitBK, WQ = 64;
+  constexpr int WGQ = BQ / WQ, TI = WP / 16, TJ = WQ / 16;
+  static_assert((BP / WP) * (BQ / WQ) == NW && WP % 16 == 0 && BP % 64 == 0 && BQ % 64 == 0, "tile shape");
+  constexpr int AC = BP / 8, BC = BQ / 8;  // units of eight rows
+  constexpr int NA = (AC + 15) / 16, NB = (BC + 15) / 16, NC = NA + NB;  // units per thread: gy, then x
+  static_assert(NC < TJ, "one unit is staged beside each column tile after the first");
+  constexpr int BUF = wgrad_split_units<BP, BQ, MODE>();
+  constexpr bool PIX = MODE == kPix4;
+
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wp = wave / WGQ, wq = wave % WGQ;
+  const int q0 = bx * BQ, p0 = by * BP;
+  const int kbeg = bz * a.kslice;
+  const int kend = min(a.K, kbeg + a.kslice);
+  const int H = a.H, W = a.W, HW = H * W, P = a.P, Q = a.Q, C = a.C, KS = a.KS, S = a.S, PAD = a.PAD;
+  const int ohw = a.OH * a.OW;
+  const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, a.x_bytes);
+  const __amdgpu_buffer_rsrc_t gr = make_rsrc(a.gy, a.gy_bytes);
+
+  // (tap, channel) of column q (tap-major and channels last)
+  const bool perm = MODE == kTapMajor && C % 32 == 0;
+  const auto column = [&](int q, int& tap, int& c) {
+    if (perm) {
+      const int b = q >> 5, cb = (int)fdiv((uint32_t)b, a.div_kk);
+      tap = b - cb * KS * KS;
+      c = 32 * cb + (q & 31);
+    } else {
+      tap = (int)fdiv((uint32_t)q, a.div_c);
+      c = q - tap * C;
+    }
+  };
+  // This thread stages pixel t % 32 of each K-block, for gy channels p0 + 8 (t / 32 + 16 u) .. + 7 and tap columns
+  // q0 + 8 (t / 32 + 16 u) .. + 7. Tap-major and channels last: the eight columns are channels of one tap. kPix4:
+  // pixels 8 (t % 4) .. + 7 of gy channels p0 + t / 4 + 128 u and x channels q0 + t / 4 + 128 u.
+  const int tk = t & 31, tc = t >> 5;
+  uint32_t goff[NA], xoff[NB];
+  int dy[NB], dx[NB], c0[NB];
+#pragma unroll
+  for (int u = 0; u < NA; ++u) {
+    const int p = p0 + 8 * (tc + 16 * u);
+    goff[u] = (uint32_t)(PIX ? (p0 + (t >> 2) + 128 * u) * ohw * 4 : MODE == kNhwc ? p * 4 : p * ohw * 4);
+  }
+#pragma unroll
+  for (int u = 0; u < NB; ++u) {
+    const int q = q0 + 8 * (tc + 16 * u);
+    if (PIX) {
+      xoff[u] = (uint32_t)((q0 + (t >> 2) + 128 * u) * HW * 4);
+      dy[u] = dx[u] = c0[u] = 0;
+    } else if (MODE == kGeneric) {  // q = (c, ky, kx)
+      const int c = (int)fdiv((uint32_t)q, a.div_kk), r = q - c * KS * KS;
+      const int ky = (int)fdiv((uint32_t)r, a.div_ks);
+      dy[u] = ky;
+      dx[u] = r - ky * KS;
+      c0[u] = c;
+      xoff[u] = 0;
+    } else {
+      int tap, c;
+      column(q, tap, c);
+      const int ky = (int)fdiv((uint32_t)tap, a.div_ks), kx = tap - ky * KS;
+      dy[u] = q < Q ? ky - PAD : -(1 << 28);  // columns past Q gather nothing
+      dx[u] = kx - PAD;
+      c0[u] = c;
+      xoff[u] = (uint32_t)((MODE == kNhwc ? ((ky - PAD) * W + kx - PAD) * C + c : c * HW + (ky - PAD) * W + kx - PAD) * 4);
+    }
+  }
+
+  // the pixel of the K-block whose loads come next
+  uint32_t gpix = kOOB, xpix = 0, gpix4 = kOOB, xpix4 = kOOB;
+  int py = -(1 << 28), px = 0;
+  auto pixel = [&](int k0) {
+    if constexpr (PIX) {  // two runs of four pixels, each of one image and whole or past kend
+      const auto run = [&](uint32_t k, uint32_t& g, uint32_t& x) {
+        const uint32_t n = fdiv(k, a.div_ohw), r = k - n * (uint32_t)ohw;
+        g = (int)k < kend ? (n * (uint32_t)(P * ohw) + r) * 4u : kOOB;
+        x = (int)k < kend ? (n * (uint32_t)(C * HW) + r) * 4u : kOOB;
+      };
+      const uint32_t k = (uint32_t)(k0 + 8 * (t & 3));
+      run(k, gpix, xpix);
+      run(k + 4, gpix4, xpix4);
+      return;
+    }
+    const uint32_t k = (uint32_t)(k0 + tk);
+    const uint32_t n = fdiv(k, a.div_ohw), r = k - n * (uint32_t)ohw;
+    const uint32_t oy = fdiv(r, a.div_ow), ox = r - oy * (uint32_t)a.OW;
+    const bool kin = (int)k < kend;
+    py = kin ? (int)oy * S : -(1 << 28);
+    px = (int)ox * S;
+    if (MODE == kNhwc) {
+      gpix = kin ? k * (uint32_t)(P * 4) : kOOB;
+      xpix = (((n * (uint32_t)H + oy * (uint32_t)S) * (uint32_t)W + ox * (uint32_t)S) * (uint32_t)C) * 4u;
+    } else {
+      gpix = kin ? (n * (uint32_t)(P * ohw) + r) * 4u : kOOB;
+      xpix = (n * (uint32_t)(C * HW) + oy * (uint32_t)(S * W) + ox * (uint32_t)S) * 4u;
+    }
+  };
+  // Unit v of this thread: gy for v < NA, x after; units past the tile's rows (tiles of 64) belong to no thread.
+  float rv[NC][8];
+  auto mine = [&](const int v) {
+    return v < NA ? (AC % 16 == 0 || tc + 16 * v < AC) : (BC % 16 == 0 || tc + 16 * (v - NA) < BC);
+  };  // (kPix4: rows t / 4 below 64 are the threads t / 32 below 8 too)
+  auto gload = [&](const int v) {
+    float* const d = rv[v];
+    if constexpr (PIX) {
+      const bool y = v < NA;
+      const uint32_t o = y ? goff[y ? v : 0] : xoff[y ? 0 : v - NA], b0 = y ? gpix : xpix, b1 = y ? gpix4 : xpix4;
+      const float4 f0 = bload4(y ? gr : xr, b0 == kOOB ? kOOB : b0 + o, 0);
+      const float4 f1 = bload4(y ? gr : xr, b1 == kOOB ? kOOB : b1 + o, 0);
+      d[0] = f0.x, d[1] = f0.y, d[2] = f0.z, d[3] = f0.w, d[4] = f1.x, d[5] = f1.y, d[6] = f1.z, d[7] = f1.w;
+      return;
+    }
+    if (v < NA) {
+      // rows past P read other rows' values, or zeros past the tensor: their sums are not stored
+      const uint32_t o = gpix == kOOB ? kOOB : gpix + goff[v];
+      if constexpr (MODE == kNhwc) {
+        const float4 f0 = bload4(gr, o, 0), f1 = bload4(gr, o, 16);
+        d[0] = f0.x, d[1] = f0.y, d[2] = f0.z, d[3] = f0.w, d[4] = f1.x, d[5] = f1.y, d[6] = f1.z, d[7] = f1.w;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) d[e] = bload(gr, o, (uint32_t)(e * ohw * 4));
+      }
+      return;
+    }
+    const int u = v - NA;
+    if constexpr (MODE == kGeneric) {
+      int c = c0[u], ky = dy[u], kx = dx[u];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int iy = py + ky - PAD, ix = px + kx - PAD;
+        const bool ok = (c < C) & ((unsigned)iy < (unsigned)H) & ((unsigned)ix < (unsigned)W);
+        d[e] = bload(xr, ok ? xpix + (uint32_t)((c * HW + (ky - PAD) * W + kx - PAD) * 4) : kOOB, 0);
+        const bool ox = ++kx == KS;
+        kx = ox ? 0 : kx;
+        ky += ox;
+        const bool oy = ky == KS;
+        ky = oy ? 0 : ky;
+        c += oy;
+      }
+    } else {
+      const bool ok = ((unsigned)(py + dy[u]) < (unsigned)H) & ((unsigned)(px + dx[u]) < (unsigned)W);
+      const uint32_t o = ok ? xpix + xoff[u] : kOOB;
+      if constexpr (MODE == kNhwc) {
+        const float4 f0 = bload4(xr, o, 0), f1 = bload4(xr, o, 16);
+        d[0] = f0.x, d[1] = f0.y, d[2] = f0.z, d[3] = f0.w, d[4] = f1.x, d[5] = f1.y, d[6] = f1.z, d[7] = f1.w;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) d[e] = bload(xr, o, (uint32_t)(e * HW * 4));
+      }
+    }
+  };
+  auto sstore = [&](const int v, const int buf) {
+    uint32_t h[4], m[4], l[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) split_bf16(rv[v][2 * e], rv[v][2 * e + 1], h[e], m[e], l[e]);
+    const int u = v < NA ? v : v - NA, c = tc + 16 * u;
+    const int term = PIX ? 4 * ((v < NA ? BP : BQ) + 4) : (v < NA ? AC : BC) * BK;  // units from one term to the next
+    uint4* const o = lds + buf * BUF + (v < NA ? 0 : 3 * (PIX ? 4 * (BP + 4) : AC * BK)) +
+                     (PIX ? (t & 3) * (term / 4) + (t >> 2) + 128 * u : c * BK + (tk ^ (4 * (c & 1))));
+    if (mine(v)) {
+      o[0] = make_uint4(h[0], h[1], h[2], h[3]);
+      o[term] = make_uint4(m[0], m[1], m[2], m[3]);
+      o[2 * term] = make_uint4(l[0], l[1], l[2], l[3]);
+    }
+  };
+
+  omt_f32x4 acc[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[i][j] = omt_f32x4{0.f, 0.f, 0.f, 0.f};
+  // MFMA operands: lane l holds row l % 16 and k 8 (l / 16) .. + 7. In the transposing read lane j of a group of 16
+  // reads k j / 4 of the four, rows 4 (j % 4) .. + 3 (unit c & 1 = j % 4 / 2, half j % 2).
+  const int grp = lane >> 4, j16 = lane & 15, cb = (j16 >> 1) & 1;
+  const int rd = (cb * BK + 8 * grp + 4 * cb + (j16 >> 2)) * 16 + 8 * (j16 & 1);  // bytes; the second four k: ^ 64
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  struct Frag { s16x4 lo, hi; };
+  // operand rows r0 .. r0 + 15 of term z: gy's (y) or x's
+  const auto frag = [&](const int buf, const bool y, const int z, const int r0) {
+    if constexpr (PIX)
+      return __builtin_bit_cast(omt_bf16x8, lds[buf * BUF + (y ? 0 : 12 * (BP + 4)) +
+                                               (4 * z + grp) * ((y ? BP : BQ) + 4) + r0 + j16]);
+    const int unit = buf * BUF + (y ? 0 : 3 * AC * BK) + (z * (y ? AC : BC) + r0 / 8) * BK;
+    const char* const b = reinterpret_cast<const char*>(lds + unit);
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    Frag f;
+    f.lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(b + rd));
+    f.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(b + (rd ^ 64)));
+    return __builtin_bit_cast(omt_bf16x8, f);
+  };
+  auto sync = [&]() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(63) & ~0xF00);  // LDS writes done; the loads in flight go on
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
+  pixel(kbeg);
+#pragma unroll
+  for (int v = 0; v < NC; ++v) gload(v);
+  pixel(kbeg + BK);
+#pragma unroll
+  for (int v = 0; v < NC; ++v) {
+    sstore(v, 0);
+    gload(v);
+  }
+  sync();
+  // x's fragments one column tile ahead where the registers allow it (a spilled load is waited for at once)
+  constexpr int NBV = TI >= 4 ? 1 : 2;
+  omt_bf16x8 av[3][TI], bv[NBV][3];
+  omt_f32x4 s[TI];  // the K-block's sums of one column tile
+  auto step = [&](int it, auto setc) {
+    constexpr int B = decltype(setc)::value;  // it & 1
+    constexpr int za[6] = {2, 0, 1, 1, 0, 0}, zb[6] = {0, 2, 1, 0, 1, 0};  // smallest partial products first
+    const auto bread = [&](int j, int z) { return frag(B, false, z, wq * WQ + 16 * j); };
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+#pragma unroll
+      for (int i = 0; i < TI; ++i) av[za[z]][i] = frag(B, true, za[z], wp * WP + 16 * i);
+      bv[0][zb[z]] = bread(0, zb[z]);
+    }
+    pixel(kbeg + (it + 2) * BK);
+    // Beside column tile j's MFMAs: the staging of unit j - 1 of the next K-block, and that unit's loads two blocks on.
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+#pragma unroll
+      for (int z = 0; z < 3; ++z) {
+        if (NBV == 2 && j + 1 < TJ) bv[(j + 1) % NBV][zb[z]] = bread(j + 1, zb[z]);
+        if (NBV == 1 && j > 0) bv[0][zb[z]] = bread(j, zb[z]);
+      }
+#pragma unroll
+      for (int i = 0; i < TI; ++i) s[i] = omt_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int z = 0; z < 6; ++z)
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+          s[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[za[z]][i], bv[j % NBV][zb[z]], s[i], 0, 0, 0);
+      if (j >= 1 && j - 1 < NC) {
+        sstore(j - 1, B ^ 1);
+        gload(j - 1);
+      }
+#pragma unroll
+      for (int i = 0; i < TI; ++i) acc[i][j] += s[i];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    sync();
+  };
+  int it = 0;
+  for (; it + 1 < nk; it += 2) {  // whole pairs: see conv_gather_split_kernel
+    step(it, std::integral_constant<int, 0>{});
+    step(it + 1, std::integral_constant<int, 1>{});
+  }
+  if (it < nk) step(it, std::integral_constant<int, 0>{});
+
+  float* const fl = reinterpret_cast<float*>(lds);
+  if (split_redo<TI, TJ, NW>(acc, wave, lane, reinterpret_cast<uint32_t*>(lds))) {
+    // the fp32 tile is the work of four waves; a barrier waits for the waves that have not ended
+    if (wave >= 4) return;
+    constexpr int FP = BP / 64, FQ = BQ / 32;
+    static_assert(wgrad_lds_floats<64, 32>() <= 8 * BUF && wgrad_nhwc_lds_floats<64, 32>() <= 8 * BUF, "fp32 tile's LDS");
+#pragma unroll 1
+    for (int f = 0; f < FP * FQ; ++f) {
+      int q = q0 + 32 * (f % FQ);
+      if (q >= Q) continue;
+      if (perm) {
+        int tap, c;
+        column(q, tap, c);
+        q = tap * C + c;
+      }
+      if constexpr (MODE == kNhwc)
+        wgrad_nhwc_tile<64, 32, 16, 32, 1>(a, q / 32, by * FP + f / FQ, bz, fl);
+      else
+        wgrad_tile<64, 32, 16, 32, MODE, 1>(a, q / 32, by * FP + f / FQ, bz, fl);
+      __syncthreads();
+    }
+    return;
+  }
+  // store in the [co][ci][ky][kx] order of the weight gradient (tap-major columns are permuted back; channels last
+  // they are its order)
+  float* out = a.out + (int64_t)bz * P * Q;
+#pragma unroll
+  for (int j = 0; j < TJ; ++j) {
+    const int q = q0 + wq * WQ + 16 * j + j16;
+    if (q >= Q) continue;
+    int col = q;
+    if (MODE == kTapMajor || MODE == kNhwc) {
+      int tap, c;
+      column(q, tap, c);
+      col = MODE == kNhwc ? q : c * KS * KS + tap;
+    }
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        const int p = p0 + wp * WP + 16 * i + 4 * grp + r4;
+        if (p < P) out[(int64_t)p * Q + col] = acc[i][j][r4];
+      }
+  }
+}
+
+template <int BP, int BQ, int WP, int MODE>
+__global__ void __launch_bounds__(kSplitNT, 2) conv_wgrad_split_kernel(const WgradArgs a) {
+  __shared__ __attribute__((aligned(16))) uint4 lds[2 * wgrad_split_units<BP, BQ, MODE>()];
+  const TileId t = xcd_block_tile(kTileGroup);
+  wgrad_split_tile<BP, BQ, WP, MODE>(a, t.x, t.y, t.z, lds);
+}
+
 // Grad input and grad weight of one convolution in one launch (omt_conv_bwd), both on 64 x 64 tiles: the first
 // gx * gy * gz workgroups run grad-input tiles, the rest grad-weight tiles over wx * wy * wz (each part through the
 // XCD tile mapping). On late,
@@ -2240,6 +2569,7 @@ static int pick_tile(const Tile (&tiles)[N], int64_t P, int64_t Q, int64_t z, in
   double best_cost = 1e300;
   for (size_t i = 0; i < N; ++i) {
     const Tile& tl = tiles[i];
+    if (tl.split) continue;
     int64_t blocks = cdiv(P, tl.bp) * cdiv(Q, tl.bq) * z;
     int64_t rounds = cdiv(blocks, slots);
     double cost = (double)rounds * tl.bp * tl.bq / tl.eff;
@@ -2302,7 +2632,34 @@ static bool split_pays(int64_t P, int64_t Q, int64_t K, int64_t z) {
 
 static const Tile kWgradTiles[] = {
     {64, 128, 32, 64, 1.00f}, {128, 64, 32, 64, 1.00f}, {64, 64, 32, 32, 0.85f}, {32, 128, 16, 64, 0.85f},
+    {128, 256, 64, 64, 2.00f, 32, 0, 1},
 };
+// The split tile (conv_wgrad_split_kernel, its shape by wgrad_split_shape): the fifth plan of the NCHW directions.
+// Channels last it is the fourth where each run of eight columns is channels of one tap (C % 8 == 0); elsewhere that
+// plan is the fp32 tile of its index.
+constexpr int kWgradSplit = 4, kWgradSplitNhwc = 3;
+static int wgrad_split_tile_of(int dir) { return dir == OMT_DIR_WGRAD_NHWC ? kWgradSplitNhwc : kWgradSplit; }
+static bool wgrad_is_split(int dir, const omt_conv_geo* g, int tile) {
+  return tile == wgrad_split_tile_of(dir) && (dir != OMT_DIR_WGRAD_NHWC || g->ci % 8 == 0);
+}
+// Its shape for P rows and Q columns: the least padded work over the shapes' relative rates (a 64-high or 64-wide tile
+// splits each staged value for half as many products).
+struct WgradSplitShape {
+  int bp, bq;
+  float eff;
+};
+static const WgradSplitShape kWgradSplitShapes[] = {{128, 256, 1.f}, {256, 128, 1.f}, {128, 128, .85f}, {64, 256, .75f}, {256, 64, .75f}};
+static int wgrad_split_shape(int64_t P, int64_t Q) {
+  int best = 0;
+  double best_cost = 1e300;
+  for (int i = 0; i < 5; ++i) {
+    const WgradSplitShape& w = kWgradSplitShapes[i];
+    const double cost = (double)(cdiv(P, w.bp) * w.bp) * (double)(cdiv(Q, w.bq) * w.bq) / w.eff;
+    if (cost < best_cost * 0.999) best_cost = cost, best = i;
+  }
+  return best;
+}
+static bool wgrad_split_pays(int64_t P, int64_t Q, int64_t K) { return P * Q * K >= ((int64_t)1 << 30); }
 
 template <int MODE, bool BN>
 static void gather_dispatch(int ti, const GatherArgs& a, dim3 grid, hipStream_t s) {
@@ -2662,14 +3019,21 @@ static const omt_conv_geo* plan_geo(const omt_conv_geo* g, omt_conv_geo& tmp) {
   return &tmp;
 }
 
-// Wgrad split: about four waves of workgroups per CU over the tiles, each slice at least four K-blocks long.
+// Wgrad split: about four waves of workgroups per CU over the tiles, each slice at least four K-blocks long; the split
+// tile, which holds a CU alone, as many slices as keep one workgroup per CU, and no more partials than the allocation-free grad weight's
+// scratch holds.
 struct WgradPlan {
   int tile;
   int64_t slices, kslice;
 };
 // The estimate's slice count for tile ti.
-static int64_t wgrad_model_slices(const omt_conv_geo* g, int ti) {
+static int64_t wgrad_model_slices(const omt_conv_geo* g, int ti, int dir) {
   const int64_t P = g->co, Q = g->ci * g->ks * g->ks, K = g->n * g->oh * g->ow;
+  if (wgrad_is_split(dir, g, ti)) {
+    const WgradSplitShape& w = kWgradSplitShapes[wgrad_split_shape(P, Q)];
+    const int64_t tiles = cdiv(P, w.bp) * cdiv(Q, w.bq);
+    return std::max<int64_t>(1, std::min<int64_t>({kCUs / tiles, cdiv(K, 64 * 4), OMT_NOALLOC_SCRATCH_BYTES / (P * Q * 4)}));
+  }
   const Tile& tl = kWgradTiles[ti];
   const int64_t tiles = cdiv(P, tl.bp) * cdiv(Q, tl.bq);
   return std::max<int64_t>(1, std::min<int64_t>(cdiv(kCUs * 4, tiles), cdiv(K, 64 * 4)));
@@ -2684,8 +3048,9 @@ static WgradPlan wgrad_plan(const omt_conv_geo* g, int dir = OMT_DIR_WGRAD) {
     ti = cp.tile;
     slices = std::max<int64_t>(1, std::min<int64_t>(cp.slices, cdiv(K, 64)));
   } else {
-    ti = pick_tile(kWgradTiles, P, Q, 1, kCUs * 2);
-    slices = wgrad_model_slices(g, ti);
+    const int sp = wgrad_split_tile_of(dir);
+    ti = wgrad_split_pays(P, Q, K) && wgrad_is_split(dir, g, sp) ? sp : pick_tile(kWgradTiles, P, Q, 1, kCUs * 2);
+    slices = wgrad_model_slices(g, ti, dir);
   }
   const int64_t kslice = cdiv(cdiv(K, slices), 64) * 64;
   return {ti, cdiv(K, kslice), kslice};
@@ -2698,6 +3063,17 @@ static void wgrad_dispatch(int ti, const WgradArgs& a, dim3 grid, hipStream_t s)
     case 1: hipLaunchKernelGGL((conv_wgrad_kernel<128, 64, 32, 64, MODE, 1>), grid, dim3(256), 0, s, a); break;
     case 2: hipLaunchKernelGGL((conv_wgrad_kernel<64, 64, 32, 32, MODE, 2>), grid, dim3(256), 0, s, a); break;
     default: hipLaunchKernelGGL((conv_wgrad_kernel<32, 128, 16, 64, MODE, 2>), grid, dim3(256), 0, s, a); break;
+  }
+}
+
+template <int MODE>
+static void wgrad_split_dispatch(const WgradArgs& a, dim3 grid, hipStream_t s) {
+  switch (wgrad_split_shape(a.P, a.Q)) {
+    case 0: hipLaunchKernelGGL((conv_wgrad_split_kernel<128, 256, 64, MODE>), grid, dim3(kSplitNT), 0, s, a); break;
+    case 1: hipLaunchKernelGGL((conv_wgrad_split_kernel<256, 128, 64, MODE>), grid, dim3(kSplitNT), 0, s, a); break;
+    case 2: hipLaunchKernelGGL((conv_wgrad_split_kernel<128, 128, 32, MODE>), grid, dim3(kSplitNT), 0, s, a); break;
+    case 3: hipLaunchKernelGGL((conv_wgrad_split_kernel<64, 256, 32, MODE>), grid, dim3(kSplitNT), 0, s, a); break;
+    default: hipLaunchKernelGGL((conv_wgrad_split_kernel<256, 64, 32, MODE>), grid, dim3(kSplitNT), 0, s, a); break;
   }
 }
 
@@ -2741,7 +3117,7 @@ static bool cached_plan(int dir, const omt_conv_geo* g, omt_conv_plan* p) {
 }
 static bool wgrad_dir(int dir) { return dir == OMT_DIR_WGRAD || dir == OMT_DIR_WGRAD_NHWC; }
 static int num_tiles(int dir) {
-  if (wgrad_dir(dir)) return (int)(sizeof(kWgradTiles) / sizeof(kWgradTiles[0]));
+  if (wgrad_dir(dir)) return dir == OMT_DIR_WGRAD_NHWC ? kWgradSplitNhwc + 1 : kWgradSplit + 1;
   return dir == OMT_DIR_FWD_NHWC || dir == OMT_DIR_DGRAD_NHWC ? kNhwcTiles : 3 * kNGather;
 }
 
@@ -3225,17 +3601,28 @@ static dim3 wgrad_prepare(const omt_conv_geo* g, const float* x, const float* gy
   a.step_oy = (int)((64 / g->ow) % g->oh);
   a.step_n = (int)((64 / g->ow) / g->oh);
   const Tile& tl = kWgradTiles[pl.tile];
-  return dim3((unsigned)cdiv(a.Q, tl.bq), (unsigned)cdiv(a.P, tl.bp), (unsigned)pl.slices);
+  const bool split = wgrad_is_split(dir, g, pl.tile);
+  const WgradSplitShape& sh = kWgradSplitShapes[wgrad_split_shape(a.P, a.Q)];
+  return dim3((unsigned)cdiv(a.Q, split ? sh.bq : tl.bq), (unsigned)cdiv(a.P, split ? sh.bp : tl.bp), (unsigned)pl.slices);
 }
-// Tap-major column order of a grad-weight launch: each wave's BQ / 4 staged columns share one tap.
+// Tap-major column order of a grad-weight launch: each wave's BQ / 4 staged columns share one tap (split tile: its
+// units of eight columns do).
 static bool wgrad_uses_tap_major(const omt_conv_geo* g, const WgradPlan& pl) {
+  if (pl.tile == kWgradSplit) return g->ci % 8 == 0;
   return g->ci % (kWgradTiles[pl.tile].bq / 4) == 0;
 }
 // The grad-weight GEMM of a plan in its loader mode: 16-byte loads of four reduction pixels for 1x1 stride-1 unpadded
 // layers whose planes are a multiple of 4 (kPix4), else one pixel per lane in tap-major or channel-major order.
 static void launch_wgrad_gemm(const omt_conv_geo* g, const WgradPlan& pl, const WgradArgs& a, dim3 grid,
                               hipStream_t s) {
-  if (g->ks == 1 && g->stride == 1 && g->pad == 0 && (g->oh * g->ow) % 4 == 0)
+  const bool pix4 = g->ks == 1 && g->stride == 1 && g->pad == 0 && (g->oh * g->ow) % 4 == 0;
+  if (pl.tile == kWgradSplit && pix4)
+    wgrad_split_dispatch<kPix4>(a, grid, s);
+  else if (pl.tile == kWgradSplit && wgrad_uses_tap_major(g, pl))
+    wgrad_split_dispatch<kTapMajor>(a, grid, s);
+  else if (pl.tile == kWgradSplit)
+    wgrad_split_dispatch<kGeneric>(a, grid, s);
+  else if (pix4)
     wgrad_dispatch<kPix4>(pl.tile, a, grid, s);
   else if (wgrad_uses_tap_major(g, pl))
     wgrad_dispatch<kTapMajor>(pl.tile, a, grid, s);
@@ -3764,7 +4151,9 @@ static int conv_wgrad_nhwc_one(const omt_conv_geo* g, const float* x, const floa
   WgradArgs a;
   WgradPlan pl;
   const dim3 grid = wgrad_prepare(g, x, gy, gw, workspace, a, pl, OMT_DIR_WGRAD_NHWC);
-  if (g->ci % 4 == 0)
+  if (wgrad_is_split(OMT_DIR_WGRAD_NHWC, g, pl.tile))
+    wgrad_split_dispatch<kNhwc>(a, grid, s);
+  else if (g->ci % 4 == 0)
     wgrad_nhwc_dispatch<false>(pl.tile, a, grid, s);
   else
     wgrad_nhwc_dispatch<true>(pl.tile, a, grid, s);
@@ -3895,12 +4284,15 @@ std::vector<omt_conv_plan> tune_candidates(int dir, const omt_conv_geo* g, int n
   if (wgrad_dir(dir)) {
     const int64_t K = g->n * g->oh * g->ow, kmax = cdiv(K, 64);
     for (int t = 0; t < ntile; ++t) {
-      const int64_t base = wgrad_model_slices(g, t);
+      const bool split = wgrad_is_split(dir, g, t);
+      if (split && !wgrad_split_pays(g->co, g->ci * g->ks * g->ks, K)) continue;
+      const int64_t base = wgrad_model_slices(g, t, dir);
       int64_t last = -1;
       for (double m : {0.25, 0.5, 1.0, 2.0}) {
+        if (split) m *= 2;  // of whole rounds of workgroups: half a round to four
         const int64_t sl = std::max<int64_t>(1, std::min<int64_t>(kmax, (int64_t)(base * m + 0.5)));
         const int64_t eff = cdiv(K, cdiv(cdiv(K, sl), 64) * 64);
-        if (eff == last || eff * g->co * g->ci * g->ks * g->ks * 4 > ((int64_t)512 << 20)) continue;
+        if (eff == last || eff * g->co * g->ci * g->ks * g->ks * 4 > (split ? (int64_t)OMT_NOALLOC_SCRATCH_BYTES : (int64_t)512 << 20)) continue;
         last = eff;
         out.push_back({t, (int32_t)eff});
       }
@@ -3960,7 +4352,9 @@ std::vector<omt_conv_plan> tune_candidates(int dir, const omt_conv_geo* g, int n
 }
 
 // Whether a plan runs a split tile.
-bool split_plan(int dir, const omt_conv_plan& p) { return !wgrad_dir(dir) && gtile(p.tile).split; }
+bool split_plan(int dir, const omt_conv_plan& p, const omt_conv_geo* g) {
+  return wgrad_dir(dir) ? wgrad_is_split(dir, g, p.tile) : gtile(p.tile).split != 0;
+}
 
 bool forcing() {
   for (const auto* f : t_force)
@@ -4099,7 +4493,7 @@ OMT_EXPORT int omt_conv_autotune(int dir, const omt_conv_geo* g, int max_tiles, 
   const std::vector<omt_conv_plan> cands = tune_candidates(dir, g, ntile);
   if (cands.empty()) return fail(OMT_UNSUPPORTED, "omt_conv_autotune: no candidate plan");
 
-  const bool random = std::any_of(cands.begin(), cands.end(), [&](const omt_conv_plan& c) { return split_plan(dir, c); });
+  const bool random = std::any_of(cands.begin(), cands.end(), [&](const omt_conv_plan& c) { return split_plan(dir, c, g); });
   ForceGuard guard;
   size_t ws_bytes = 0;
   for (const omt_conv_plan& c : cands) {
@@ -4172,7 +4566,7 @@ OMT_EXPORT int omt_conv_autotune_bwd(const omt_conv_geo* g, int max_tiles, void*
     for (const omt_conv_plan& d : ds)
       for (const omt_conv_plan& w : wsv) cands.push_back({d, w});
   }
-  const bool random = split_plan(OMT_DIR_DGRAD, dsep) || split_plan(OMT_DIR_WGRAD, wsep);
+  const bool random = split_plan(OMT_DIR_DGRAD, dsep, g) || split_plan(OMT_DIR_WGRAD, wsep, g);
   ForceGuard guard;
   size_t ws_bytes = 0;
   for (const auto& c : cands) {

@@ -97,3 +97,73 @@ def test_split_tile_falls_back_on_values_it_cannot_split(cuda, ops, kind):
                 assert np.abs(a[f].astype(np.float64) - b[f]).max() <= 2 * 432 * 2.0 ** -24 * scale
     finally:
         ops.clear_conv_plans()
+
+
+WSPLIT, WSPLIT_NHWC, WFP32 = 4, 3, 2  # grad-weight tiles
+# rows around 64, 128 and 256, columns around 64, 128 and 256 (all five tile shapes); reductions that end inside a
+# K-block; the orders by channels: % 32 (columns by 32 channels), % 8 (tap-major), others (element by element); 1x1
+# planes of a multiple of 4 that is none of 8 (runs of four pixels that change image)
+WSHAPES = [
+    (3, 32, 64, 9, 11, 3, 1, 1), (2, 64, 128, 8, 8, 3, 1, 1), (2, 40, 130, 9, 9, 3, 2, 1), (1, 13, 65, 12, 10, 3, 1, 1),
+    (3, 130, 256, 6, 6, 1, 1, 0), (5, 64, 300, 2, 6, 1, 1, 0), (2, 72, 260, 7, 7, 1, 1, 0), (1, 3, 48, 30, 31, 7, 2, 3),
+    (2, 256, 64, 5, 5, 1, 1, 0), (1, 8, 16, 3, 3, 3, 1, 1),
+]
+
+
+@pytest.mark.parametrize("shape", WSHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_split_grad_weight_is_as_exact_as_the_fp32_tile(cuda, ops, shape):
+    """Both memory formats, 1 and 3 K slices, against the float64 oracle: off by no more than the fp32 tile, or one
+    rounding of the result."""
+    n, ci, co, h, w, ks, s, p = shape
+    rng = np.random.default_rng(sum(shape) + 1)
+    x, wt = rnd(rng, n, ci, h, w), rnd(rng, co, ci, ks, ks)
+    gy = rnd(rng, *orc.conv_fwd(x, wt, None, s, p).shape)
+    ref = orc.conv_wgrad(x, gy, ks, s, p)
+    try:
+        for d, tile, fn in (("wgrad", WSPLIT, ops.conv2d_wgrad), ("wgrad_nhwc", WSPLIT_NHWC, ops.conv2d_wgrad_nhwc)):
+            if d == "wgrad_nhwc" and co % 4:
+                continue  # not covered channels-last
+            t = [torch.from_numpy(a).to(cuda) for a in (x, gy)]
+            t = [a.contiguous(memory_format=_CL) for a in t] if d == "wgrad_nhwc" else t
+            for slices in (1, 3):
+                ops.set_conv_plan(d, x.shape, wt.shape, s, p, WFP32, slices)
+                e32 = orc.rel_l2(fn(t[0], t[1], ks, s, p).contiguous().cpu().numpy(), ref)
+                ops.set_conv_plan(d, x.shape, wt.shape, s, p, tile, slices)
+                err = orc.rel_l2(fn(t[0], t[1], ks, s, p).contiguous().cpu().numpy(), ref)
+                assert err <= max(e32, 2.0 ** -24), (d, slices, err, e32)
+    finally:
+        ops.clear_conv_plans()
+
+
+@pytest.mark.parametrize("shape", [(2, 32, 70, 9, 9, 3, 1, 1), (2, 24, 70, 9, 9, 3, 1, 1), (2, 12, 64, 9, 9, 3, 1, 1),
+                                   (2, 70, 68, 8, 8, 1, 1, 0)], ids=lambda s: "x".join(map(str, s)))
+def test_split_grad_weight_falls_back_on_values_it_cannot_split(cuda, ops, shape):
+    """Every column order of the tile: an infinity and a NaN reach the same weights as through the fp32 tile, and
+    inputs whose low terms underflow give the fp32 tile's sums to the bit (both sum each K slice in the same order)."""
+    n, ci, co, h, w, ks, s, p = shape
+    rng = np.random.default_rng(sum(shape) + 2)
+    x, gy = rnd(rng, n, ci, h, w), rnd(rng, n, co, h + 2 * p - ks + 1, w + 2 * p - ks + 1)
+    try:
+        for kind in ("special", "tiny"):
+            a = x * np.float32(2.0 ** -112) if kind == "tiny" else x.copy()
+            if kind == "special":
+                a[0, 3, 4, 4], a[1, 5, 2, 2] = np.inf, np.nan
+            for d, tile, fn in (("wgrad", WSPLIT, ops.conv2d_wgrad), ("wgrad_nhwc", WSPLIT_NHWC, ops.conv2d_wgrad_nhwc)):
+                if d == "wgrad_nhwc" and co % 4:
+                    continue
+                t = [torch.from_numpy(v).to(cuda) for v in (a, gy)]
+                t = [v.contiguous(memory_format=_CL) for v in t] if d == "wgrad_nhwc" else t
+                got = []
+                for tl in (tile, WFP32):
+                    ops.set_conv_plan(d, x.shape, (co, ci, ks, ks), s, p, tl, 2)
+                    got.append(fn(t[0], t[1], ks, s, p).contiguous().cpu().numpy())
+                assert np.array_equal(np.isnan(got[0]), np.isnan(got[1]))
+                assert np.array_equal(np.isinf(got[0]), np.isinf(got[1]))
+                f = np.isfinite(got[1])
+                if kind == "tiny":
+                    assert np.array_equal(got[0], got[1])
+                else:  # both within K 2^-24 relative of the exact sums (K = 162 products)
+                    scale = np.sqrt((got[1][f].astype(np.float64) ** 2).mean())
+                    assert np.abs(got[0][f].astype(np.float64) - got[1][f]).max() <= 2 * 162 * 2.0 ** -24 * scale
+    finally:
+        ops.clear_conv_plans()

@@ -76,6 +76,7 @@ struct Phase {
   int woff;               // offset of this phase's [P][K] weights (floats)
   int ky0, kx0;           // grad input read straight from w: the phase's first filter tap
   int soff, snkb;         // split tile: the phase's first 16-byte unit of the packed filter, and its K-blocks
+  FastDiv div_sw, div_sh; // window tile: OW + KW - 1 (a row of staged pixels), OH + KH - 1 (an image's rows of them)
   FastDiv div_ohw, div_ow, div_kk, div_kw;
 };
 
@@ -104,6 +105,7 @@ struct GatherArgs {
   uint32_t w_rowst, w_cst, w_tst;  // wplace: bytes between A rows, consecutive channels of one tap, and taps
   const uint32_t* wsplit;  // split tile: the filter in split_pack_kernel's layout
   uint32_t wsplit_bytes;
+  int gx, gy;              // split tiles: the tile grid's extents (SplitTiles)
   float* part;           // split K: raw partials [slices][N][P][YH][YW], else null (epilogue writes y)
   int64_t part_stride;   // elements per slice
   int nhwc;              // channels-last source [N][H][W][C] and output [N][YH][YW][P] (partials likewise)
@@ -736,6 +738,7 @@ __device__ __forceinline__ void split_bf16(float x, float y, uint32_t& h, uint32
 // rows that a wave writes, so both run without bank conflicts.
 constexpr int kSplitBK = 32, kSplitRun = 16;  // K-block; channels per tap run of the tap-major order
 constexpr int kSplitNT = 512;                 // threads of a workgroup (one per CU: two waves per SIMD)
+constexpr int kSplitBQ = 256;                 // columns of a gather tile
 
 // The filter, packed for the split tile: for each phase, tile of BP rows and K-block, the K-block's units in LDS
 // order, rows past P and k past K zero. One thread per (row, 8 k): three units.
@@ -778,6 +781,28 @@ __global__ void __launch_bounds__(256) split_pack_kernel(const GatherArgs a, uin
   o[8 * BP] = make_uint4(l[0], l[1], l[2], l[3]);
 }
 
+// The tiles of one workgroup: every gridDim.x-th of a grid of ntiles = gx gy gz tiles (a.gx, a.gy), in xcd_tile's order.
+// A launch of one phase and no K split (gz 1) has at most one workgroup per CU, which runs its tiles as one pipeline:
+// the next tile's first K-blocks are loaded and staged under the current tile's last MFMAs, where a workgroup per tile
+// waits for its first loads, with the whole CU's LDS to itself (batch 256: 1x1 64 -> 256 channels at 56x56 350 -> 282 us,
+// 128 -> 512 at 28x28 241 -> 221). The window tile, whose tiles are longer, keeps a workgroup per tile (a next tile's
+// loads cost it its registers: 346 -> 365 us for 3x3 128 channels at 28x28).
+struct SplitTiles {
+  int pid;
+  TileId t;
+  __device__ __forceinline__ SplitTiles(const GatherArgs& a, int ntiles) : pid((int)blockIdx.x), gx(a.gx), gy(a.gy) {
+    if (pid < ntiles) t = at(ntiles);
+  }
+  __device__ __forceinline__ void next(int ntiles) {
+    pid += (int)gridDim.x;
+    if (pid < ntiles) t = at(ntiles);
+  }
+
+ private:
+  int gx, gy;
+  __device__ __forceinline__ TileId at(int ntiles) const { return xcd_tile(pid, gx, gy, ntiles / (gx * gy), kTileGroup); }
+};
+
 // Whether a workgroup's finished sums call for the fp32 tile (see above), the same answer in every thread. Uses a
 // dword of LDS per wave at `flags` that no wave still reads; returns after a barrier, with `flags` free again.
 template <int TI, int TJ, int NW>
@@ -801,6 +826,37 @@ __device__ __forceinline__ bool split_redo(const omt_f32x4 (&acc)[TI][TJ], int w
   return (all & 1u) || (all & 6u) == 4u;
 }
 
+// The outputs of a finished split gather tile. lds: row_epi_floats() per wave, free of other use.
+template <int BP, int BQ, int WP, int WQ, int MODE>
+__device__ __forceinline__ void split_epilogue(const GatherArgs& a, const Phase& ph,
+                                               const omt_f32x4 (&acc)[WP / 16][WQ / 16], int bx, int by, int zs,
+                                               int wave, int lane, float* __restrict__ lds) {
+  constexpr int WGQ = BQ / WQ, TI = WP / 16, TJ = WQ / 16;
+  const int q0 = bx * BQ, p0 = by * BP, wp = wave / WGQ, wq = wave % WGQ;
+  if constexpr (MODE == kNhwc)
+    gather_epilogue_nhwc<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane, zs);
+  else if (a.d2s && !a.part)
+    d2s_epilogue<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane);
+  else if (a.rows)
+    row_epilogue<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane, lds + wave * row_epi_floats<WQ>());
+  else
+    gather_epilogue<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane, zs);
+}
+// The tiles of one workgroup again in fp32 (split_redo asked for it on one of them), after all their split results.
+template <int BP, int BQ, int MODE>
+__device__ __forceinline__ void split_redo_tiles(const GatherArgs& a, int ntiles, int wave, float* __restrict__ lds) {
+  // the fp32 tile is the work of four waves; a barrier waits for the waves that have not ended
+  if (wave >= 4) return;
+  constexpr int FQ = BQ / 128, FP = BP / 64, FMODE = MODE == kTapMajor ? kTapInPlace : MODE;
+#pragma unroll 1
+  for (SplitTiles w(a, ntiles); w.pid < ntiles; w.next(ntiles))
+#pragma unroll 1
+    for (int f = 0; f < FP * FQ; ++f) {
+      gather_tile<64, 128, 32, 64, 16, FMODE, false, 2>(a, w.t.x * FQ + f % FQ, w.t.y * FP + f / FQ, w.t.z, lds);
+      __syncthreads();
+    }
+}
+
 // Units between consecutive k groups of the staged source: channels last, four more than its rows, so that the four
 // groups that a quad of lanes writes for one pixel fall on disjoint banks.
 template <int BQ, int MODE>
@@ -808,79 +864,102 @@ constexpr int split_bstride() { return BQ + (MODE == kNhwc ? 4 : 0); }
 template <int BP, int BQ, int MODE>
 constexpr int split_lds_units() { return 12 * (BP + split_bstride<BQ, MODE>()); }  // of one buffer
 
-// One workgroup's split-bf16 tile: gather_tile's source loaders (kGeneric, kTapMajor, kNhwc), plans and epilogues. The
+// One workgroup's split-bf16 tiles: gather_tile's source loaders (kGeneric, kTapMajor, kNhwc), plans and epilogues. The
 // filter comes packed (split_pack_kernel) and goes to LDS directly; the source is split as it is staged. K-blocks are
 // two runs of 16 k: in the tap-major orders a run is 16 channels of one tap (C % 16 == 0), so that the K order does
 // not depend on whether C is a multiple of 32. Two LDS buffers: while the MFMAs of K-block b run, the wave splits and
-// stores its part of b + 1 between them, b + 1's filter is on its way to LDS, and b + 2's source is being loaded.
+// stores its part of b + 1 between them, b + 1's filter is on its way to LDS, and b + 2's source is being loaded; past
+// a tile's last K-block these are the next tile's.
 template <int BP, int BQ, int WP, int WQ, int MODE>
-__device__ __forceinline__ void gather_split_tile(const GatherArgs& a, const int bx, const int by, const int bz,
-                                                  uint4* __restrict__ lds) {
+__device__ __forceinline__ void gather_split_tiles(const GatherArgs& a, const int ntiles, uint4* __restrict__ lds) {
   constexpr int NT = kSplitNT, NW = NT / 64, BK = kSplitBK, RUN = kSplitRun;
   constexpr int WGQ = BQ / WQ;
   static_assert((BP / WP) * (BQ / WQ) == NW && WP % 16 == 0 && WQ == 64 && BQ == NT / 2, "tile shape");
   constexpr int TI = WP / 16, TJ = WQ / 16;
   constexpr int BS = split_bstride<BQ, MODE>(), BUF = split_lds_units<BP, BQ, MODE>();
 
-  const int zs = bz / a.nphase;  // K slice
-  const Phase ph = a.ph[bz - zs * a.nphase];
-  const int q0 = bx * BQ, p0 = by * BP;
-  if (q0 >= ph.Q) return;  // this phase has fewer pixel tiles than the largest one
+  SplitTiles cur(a, ntiles);
+  const int zs = cur.t.z / a.nphase;  // K slice
+  const Phase ph = a.ph[cur.t.z - zs * a.nphase];
+  if (cur.t.x * BQ >= ph.Q) return;  // this phase has fewer pixel tiles than the largest one
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wp = wave / WGQ, wq = wave % WGQ;
   const int KH = ph.KH, KW = ph.KW, K = ph.K, KK = KH * KW;
   const int H = a.H, W = a.W, HW = H * W, C = a.C;
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, a.x_bytes);
+  const int kbeg = zs * a.kslice, kend = min(K, kbeg + a.kslice);
+  // an empty slice runs one K-block past K, all zeros, and writes its (zero) tile
+  const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 1;
 
   // This thread's part of a K-block of the source: k rbase .. rbase + 15 of pixel t % BQ, or, channels last, k 8 cg ..
   // 8 cg + 7 of pixels t / 4 and t / 4 + 128 (four lanes read one pixel's contiguous 128 bytes).
-  // lb0: byte offset of x[n][0][iy][ix] (channels last: of the first of its channels of the pixel)
+  // The source loader's place: tile, K-block, lb0: byte offset of x[n][0][iy][ix] (channels last: of the first of its
+  // channels of the pixel), and in the tap-major orders the tap (rky, rkx) and first channel rc of its run.
   constexpr int NPX = MODE == kNhwc ? 2 : 1;
   const int run = MODE == kNhwc ? (t & 3) >> 1 : __builtin_amdgcn_readfirstlane(t / BQ);
   const int rbase = RUN * run, cg = t & 3;
-  int iy[NPX], ix[NPX];
+  int iy[NPX], ix[NPX], rc = 0, rky = 0, rkx = 0, bk = kbeg;
   uint32_t lb0[NPX];
+  SplitTiles bt = cur;
+  auto bstart = [&]() {
 #pragma unroll
-  for (int j = 0; j < NPX; ++j) {
-    const int q = q0 + (MODE == kNhwc ? t / 4 + 128 * j : t % BQ);
-    iy[j] = ix[j] = -(1 << 28);  // pixels past Q gather nothing
-    lb0[j] = kOOB;
-    if (q < ph.Q) {
-      const uint32_t ohw = (uint32_t)(ph.OH * ph.OW);
-      const uint32_t n = fdiv((uint32_t)q, ph.div_ohw), r = (uint32_t)q - n * ohw;
-      const uint32_t oy = fdiv(r, ph.div_ow), ox = r - oy * (uint32_t)ph.OW;
-      iy[j] = (int)oy * ph.S - ph.PH;
-      ix[j] = (int)ox * ph.S - ph.PW;
-      lb0[j] = MODE == kNhwc ? (uint32_t)((((int)n * H + iy[j]) * W + ix[j]) * C * 4 + 32 * (cg & 1))
-                             : (uint32_t)(((int)n * C * HW + iy[j] * W + ix[j]) * 4);
+    for (int j = 0; j < NPX; ++j) {
+      const int q = bt.t.x * BQ + (MODE == kNhwc ? t / 4 + 128 * j : t % BQ);
+      iy[j] = ix[j] = -(1 << 28);  // pixels past Q gather nothing
+      lb0[j] = kOOB;
+      if (bt.pid < ntiles && q < ph.Q) {
+        const uint32_t ohw = (uint32_t)(ph.OH * ph.OW);
+        const uint32_t n = fdiv((uint32_t)q, ph.div_ohw), r = (uint32_t)q - n * ohw;
+        const uint32_t oy = fdiv(r, ph.div_ow), ox = r - oy * (uint32_t)ph.OW;
+        iy[j] = (int)oy * ph.S - ph.PH;
+        ix[j] = (int)ox * ph.S - ph.PW;
+        lb0[j] = MODE == kNhwc ? (uint32_t)((((int)n * H + iy[j]) * W + ix[j]) * C * 4 + 32 * (cg & 1))
+                               : (uint32_t)(((int)n * C * HW + iy[j] * W + ix[j]) * 4);
+      }
     }
-  }
-
-  const int kbeg = zs * a.kslice, kend = min(K, kbeg + a.kslice);
-  const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;  // an empty slice still writes its (zero) tile
-  // tap-major orders: the tap (rky, rkx) and first channel rc of this thread's run of the next K-block gload reads
-  int rc = 0, rky = 0, rkx = 0;
-  if constexpr (MODE != kGeneric) {
-    const uint32_t kb = (uint32_t)(kbeg + rbase);
-    const int tap = (int)fdiv(kb, a.div_c);
-    rc = (int)kb - tap * C;
-    rky = (int)fdiv((uint32_t)tap, ph.div_kw);
-    rkx = tap - rky * KW;
-  }
-
-  float rb[2][RUN];  // two register sets: source loads two K-blocks ahead of the MFMAs
-  auto gload = [&](int k0, const int set) {
+    bk = kbeg;
+    if constexpr (MODE != kGeneric) {
+      const uint32_t kb = (uint32_t)(kbeg + rbase);
+      const int tap = (int)fdiv(kb, a.div_c);
+      rc = (int)kb - tap * C;
+      rky = (int)fdiv((uint32_t)tap, ph.div_kw);
+      rkx = tap - rky * KW;
+    }
+  };
+  auto bnext = [&]() {
+    bk += BK;
+    if (bk >= kbeg + nk * BK) {
+      bt.next(ntiles);
+      bstart();
+      return;
+    }
+    if constexpr (MODE != kGeneric) {
+      rc += BK;  // the next K-block's run; 32 channels on may cross two taps (C of 16)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const bool over = rc >= C;
+        rc -= over ? C : 0;
+        rkx += over;
+        const bool wrap = rkx == KW;
+        rkx = wrap ? 0 : rkx;
+        rky += wrap;
+      }
+    }
+  };
+  // Four of this thread's sixteen source values of K-block bk: channels last, half of one pixel's eight.
+  float rb[RUN];
+  auto gload = [&](const int quarter) {
     if constexpr (MODE == kGeneric) {
-      const uint32_t kb = (uint32_t)(k0 + rbase);
+      const uint32_t kb = (uint32_t)(bk + rbase + 4 * quarter);
       int c = (int)fdiv(kb, ph.div_kk);
       const uint32_t rr = kb - (uint32_t)c * (uint32_t)KK;
       int ky = (int)fdiv(rr, ph.div_kw);
       int kx = (int)rr - ky * KW;
 #pragma unroll
-      for (int e = 0; e < RUN; ++e) {
-        const bool ok = (k0 + rbase + e < K) & ((unsigned)(iy[0] + ky) < (unsigned)H) & ((unsigned)(ix[0] + kx) < (unsigned)W);
-        rb[set][e] = bload(xr, ok ? lb0[0] + (uint32_t)((c * HW + ky * W + kx) * 4) : kOOB, 0);
+      for (int e = 0; e < 4; ++e) {
+        const bool ok = ((int)kb + e < K) & ((unsigned)(iy[0] + ky) < (unsigned)H) & ((unsigned)(ix[0] + kx) < (unsigned)W);
+        rb[4 * quarter + e] = bload(xr, ok ? lb0[0] + (uint32_t)((c * HW + ky * W + kx) * 4) : kOOB, 0);
         if (++kx == KW) {
           kx = 0;
           if (++ky == KH) {
@@ -891,57 +970,50 @@ __device__ __forceinline__ void gather_split_tile(const GatherArgs& a, const int
       }
       return;
     }
-    const bool kin = k0 + rbase < K;  // the second half of an odd last block is past K
+    const bool kin = bk + rbase < K;  // the second half of an odd last block is past K
     if constexpr (MODE == kNhwc) {
-      const uint32_t toff = (uint32_t)(((rky * W + rkx) * C + rc) * 4);
-#pragma unroll
-      for (int j = 0; j < NPX; ++j) {
-        const bool ok = kin & ((unsigned)(iy[j] + rky) < (unsigned)H) & ((unsigned)(ix[j] + rkx) < (unsigned)W);
-        const uint32_t off = ok ? lb0[j] + toff : kOOB;
-        const float4 v0 = bload4(xr, off, 0), v1 = bload4(xr, off, 16);
-        float* const d = &rb[set][8 * j];
-        d[0] = v0.x, d[1] = v0.y, d[2] = v0.z, d[3] = v0.w, d[4] = v1.x, d[5] = v1.y, d[6] = v1.z, d[7] = v1.w;
-      }
+      const int j = quarter / 2;
+      const bool ok = kin & ((unsigned)(iy[j] + rky) < (unsigned)H) & ((unsigned)(ix[j] + rkx) < (unsigned)W);
+      const float4 v = bload4(xr, ok ? lb0[j] + (uint32_t)(((rky * W + rkx) * C + rc) * 4) : kOOB, 16 * (quarter & 1));
+      float* const d = &rb[4 * quarter];
+      d[0] = v.x, d[1] = v.y, d[2] = v.z, d[3] = v.w;
     } else {
       const bool ok = kin & ((unsigned)(iy[0] + rky) < (unsigned)H) & ((unsigned)(ix[0] + rkx) < (unsigned)W);
       const uint32_t voff = ok ? lb0[0] + (uint32_t)((rky * W + rkx) * 4) : kOOB;
 #pragma unroll
-      for (int e = 0; e < RUN; ++e) rb[set][e] = bload(xr, voff, (uint32_t)((rc + e) * HW * 4));
-    }
-    rc += BK;  // the next K-block's run; 32 channels on may cross two taps (C of 16)
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const bool over = rc >= C;
-      rc -= over ? C : 0;
-      rkx += over;
-      const bool wrap = rkx == KW;
-      rkx = wrap ? 0 : rkx;
-      rky += wrap;
+      for (int e = 4 * quarter; e < 4 * quarter + 4; ++e) rb[e] = bload(xr, voff, (uint32_t)((rc + e) * HW * 4));
     }
   };
-  constexpr int NLOADS = MODE == kNhwc ? 4 : RUN;  // of one gload
+  constexpr int NLOADS = MODE == kNhwc ? 4 : RUN;  // of a K-block
 
-  // The filter's K-block kb (of the slice's first), 1 KB per instruction: BP 12 units of 16 bytes.
+  // The filter loader: K-block ak of tile at, 1 KB per instruction: BP 12 units of 16 bytes.
   const omt_u32x4 wr = rsrc_words(a.wsplit, a.wsplit_bytes);
   constexpr int AKB = BP * 12 / 64;  // 1 KB pieces
   const uint32_t alds = lds_addr(reinterpret_cast<const float*>(lds));
-  const uint32_t asrc = (uint32_t)((ph.soff + (by * ph.snkb + kbeg / BK) * 12 * BP) * 16);
-  auto aload = [&](int it, const int buf) {
+  SplitTiles at = cur;
+  int ak = 0;
+  auto aload = [&](const int buf) {
+    const uint32_t src = (uint32_t)((ph.soff + (at.t.y * ph.snkb + kbeg / BK + ak) * 12 * BP) * 16);
 #pragma unroll
     for (int i = 0; i < (AKB + NW - 1) / NW; ++i) {
       const int c = wave + NW * i;
       if (AKB % NW == 0 || c < AKB)
-        lds_load_b128s(wr, alds + (uint32_t)(buf * BUF * 16 + c * 1024), (uint32_t)(lane * 16),
-                       asrc + (uint32_t)(it * 12 * BP * 16 + c * 1024));
+        lds_load_b128s(wr, alds + (uint32_t)(buf * BUF * 16 + c * 1024), (uint32_t)(lane * 16), src + (uint32_t)(c * 1024));
+    }
+  };
+  auto anext = [&]() {  // past the last tile it stays there: its loads are not read
+    if (++ak == nk) {
+      ak = 0;
+      at.next(ntiles);
     }
   };
 
   // A quarter of this thread's source values: split four k, and store each eight as three units.
   uint32_t sh[4], sm[4], sl[4];
-  auto sstore = [&](const int quarter, const int set, const int buf) {
+  auto sstore = [&](const int quarter, const int buf) {
     const int e = 4 * quarter, u = 2 * (quarter & 1);
-    split_bf16(rb[set][e], rb[set][e + 1], sh[u], sm[u], sl[u]);
-    split_bf16(rb[set][e + 2], rb[set][e + 3], sh[u + 1], sm[u + 1], sl[u + 1]);
+    split_bf16(rb[e], rb[e + 1], sh[u], sm[u], sl[u]);
+    split_bf16(rb[e + 2], rb[e + 3], sh[u + 1], sm[u + 1], sl[u + 1]);
     if (quarter & 1) {
       const int g = MODE == kNhwc ? cg : rbase / 8 + quarter / 2;
       const int row = MODE == kNhwc ? t / 4 + 128 * (quarter / 2) : t % BQ;
@@ -953,10 +1025,6 @@ __device__ __forceinline__ void gather_split_tile(const GatherArgs& a, const int
   };
 
   omt_f32x4 acc[TI][TJ];
-#pragma unroll
-  for (int i = 0; i < TI; ++i)
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) acc[i][j] = omt_f32x4{0.f, 0.f, 0.f, 0.f};
   // Lane group grp supplies k = 8 grp .. 8 grp + 7 of both operands; the accumulator layout is that of the 16x16x4
   // fp32 instruction.
   const int la = wp * WP + (lane & 15), lb = wq * WQ + (lane & 15), grp = lane >> 4;
@@ -968,90 +1036,310 @@ __device__ __forceinline__ void gather_split_tile(const GatherArgs& a, const int
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  aload(0, 0);
-  gload(kbeg, 0);
+  aload(0);
+  anext();
+  bstart();
 #pragma unroll
-  for (int v = 0; v < 4; ++v) sstore(v, 0, 0);
-  gload(kbeg + BK, 1);
+  for (int v = 0; v < 4; ++v) gload(v);
+  bnext();
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    sstore(v, 0);
+    gload(v);
+  }
+  bnext();
   sync();
-  omt_bf16x8 av[3][TI], bv[2][3];
+  bool redo = false;
+  int buf = 0;
+#pragma unroll 1
+  for (; cur.pid < ntiles; cur.next(ntiles)) {
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) acc[i][j] = omt_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int it = 0; it < nk; ++it, buf ^= 1) {
+      constexpr int za[6] = {2, 0, 1, 1, 0, 0}, zb[6] = {0, 2, 1, 0, 1, 0};  // smallest partial products first
+      const uint4* const ab = lds + buf * BUF + grp * BP + la;
+      const uint4* const bb = lds + buf * BUF + 12 * BP + grp * BS + lb;
+      const auto bread = [&](int j, int z) { return __builtin_bit_cast(omt_bf16x8, bb[4 * z * BS + 16 * j]); };
+      omt_bf16x8 av[3][TI], bv[2][3];
+      omt_f32x4 s[2][TI];  // the K-block's sums of column tiles j and j - 1
+#pragma unroll
+      for (int z = 0; z < 3; ++z) {
+#pragma unroll
+        for (int i = 0; i < TI; ++i) av[za[z]][i] = __builtin_bit_cast(omt_bf16x8, ab[4 * za[z] * BP + 16 * i]);
+        bv[0][zb[z]] = bread(0, zb[z]);
+      }
+      aload(buf ^ 1);
+      // Column tile j's MFMAs run beside the additions of the tile before, a quarter of the staging of the next
+      // K-block, and that quarter's loads of the block after it.
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) {
+#pragma unroll
+        for (int z = 0; z < 3; ++z)
+          if (j + 1 < TJ) bv[(j + 1) & 1][zb[z]] = bread(j + 1, zb[z]);
+#pragma unroll
+        for (int i = 0; i < TI; ++i) s[j & 1][i] = omt_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int z = 0; z < 6; ++z)
+#pragma unroll
+          for (int i = 0; i < TI; ++i)
+            s[j & 1][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[za[z]][i], bv[j & 1][zb[z]], s[j & 1][i], 0, 0, 0);
+        sstore(j, buf ^ 1);
+        gload(j);
+        if (j > 0)
+#pragma unroll
+          for (int i = 0; i < TI; ++i) acc[i][j - 1] += s[(j + 1) & 1][i];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      anext();
+      bnext();
+#pragma unroll
+      for (int i = 0; i < TI; ++i) acc[i][TJ - 1] += s[(TJ - 1) & 1][i];
+      sync();
+    }
+    // the next tile's first K-block waits in buffer `buf`; the other one is free for the epilogue
+    float* const fl = reinterpret_cast<float*>(lds + (buf ^ 1) * BUF);
+    redo |= split_redo<TI, TJ, NW>(acc, wave, lane, reinterpret_cast<uint32_t*>(fl));
+    split_epilogue<BP, BQ, WP, WQ, MODE>(a, ph, acc, cur.t.x, cur.t.y, zs, wave, lane, fl);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(63) & ~0xF00);
+    __builtin_amdgcn_s_barrier();  // the next step writes that buffer
+    asm volatile("" ::: "memory");
+  }
+  static_assert(NW * row_epi_floats<WQ>() <= 4 * BUF && gather_lds_floats<64, 128, 16>() <= 8 * BUF, "LDS");
+  if (redo) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0) & ~0xF00);  // filter loads on their way to LDS
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    split_redo_tiles<BP, BQ, MODE>(a, ntiles, wave, reinterpret_cast<float*>(lds));
+  }
+}
+
+template <int BP, int BQ, int WP, int WQ, int MODE>
+__global__ void __launch_bounds__(kSplitNT, 2) conv_gather_split_kernel(const GatherArgs a, const int ntiles) {
+  __shared__ __attribute__((aligned(16))) uint4 lds[2 * split_lds_units<BP, BQ, MODE>()];
+  gather_split_tiles<BP, BQ, WP, WQ, MODE>(a, ntiles, lds);
+}
+
+// ---- split-bf16 window tiles --------------------------------------------------------------------------------------
+// Stride-1 windows of more than one tap (3x3 forward and grad input, the phases of a strided grad input, the
+// super-pixel grad input): conv_gather_split_kernel loads, splits and stages a source value once per tap, which bounds
+// it by VALU work (64 x 256 tile, 3x3: 3.7 VALU instructions per MFMA). Here a workgroup stages, for 32 channels at a
+// time, every input pixel that its 256 output pixels' windows touch, once, and all taps read it from LDS at shifted
+// addresses: a K-block per tap is then the filter's 32 x BP terms (to LDS directly, double-buffered) and MFMAs.
+// Batch 256, forward: 3x3 64 channels at 56x56 433 -> 401 us, 128 channels at 28x28 391 -> 364, 256 at 14x14 363 -> 353.
+// The staged pixels ("slots") are rows of OW + KW - 1 pixels: output row (n, oy) reads slot rows (n - n0) (OH + KH - 1)
+// + oy - oy0 + ky, where (n0, oy0) is the row of the tile's first pixel, so rows of one image share their input rows
+// and each further image adds KH - 1. The sum runs over channel blocks, then taps. Unsplit plans only (a K slice is a
+// run of taps).
+// A step (one barrier) runs two taps of a 64-high tile, whose MFMAs per tap are half as many, or one of a 128-high tile.
+constexpr int window_taps(int bp) { return 128 / bp; }
+constexpr int kWindowSlots = ((160 * 1024 / 16 - 2 * 12 * 128) / 12 - 4) / 16 * 16 + 4;  // as 160 KB of LDS hold, 4 mod 16
+
+template <int BP, int WP, int MODE>
+__device__ __forceinline__ void gather_window_tile(const GatherArgs& a, const int ntiles, uint4* __restrict__ lds) {
+  constexpr int NT = kSplitNT, NW = NT / 64, BQ = kSplitBQ, WQ = 64, BK = kSplitBK;
+  constexpr int WGQ = BQ / WQ, TI = WP / 16, TJ = WQ / 16;
+  static_assert((BP / WP) * WGQ == NW && WP % 16 == 0, "tile shape");
+  // slots of one term and group of eight channels, 4 mod 16: channels last, a quad of lanes writes the four groups of
+  // a pixel to disjoint banks
+  constexpr int NS = kWindowSlots, AT = window_taps(BP), ATAP = 12 * BP, ABUF = AT * ATAP;
+  constexpr int NU = (NS + NT / 4 - 1) / (NT / 4);  // items per thread
+  uint4* const Bs = lds + 2 * ABUF;
+
+  const TileId tile = SplitTiles(a, ntiles).t;
+  const Phase ph = a.ph[tile.z];
+  const int q0 = tile.x * BQ;
+  if (q0 >= ph.Q) return;  // this phase has fewer pixel tiles than the largest one
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wp = wave / WGQ, wq = wave % WGQ;
+  const int KW = ph.KW, KK = ph.KH * KW, H = a.H, W = a.W, HW = H * W, C = a.C;
+  const int SW = ph.OW + KW - 1, SH = ph.OH + ph.KH - 1;  // slot row length; slot rows of a whole image
+  const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, a.x_bytes);
+  const uint32_t ohw = (uint32_t)(ph.OH * ph.OW);
+  const auto pixel = [&](int q, int& n, int& oy, int& ox) {
+    n = (int)fdiv((uint32_t)q, ph.div_ohw);
+    const uint32_t r = (uint32_t)q - (uint32_t)n * ohw;
+    oy = (int)fdiv(r, ph.div_ow);
+    ox = (int)r - oy * ph.OW;
+  };
+  // This thread's items (slot, eight channels): slots t % 128 + 128 u, group t / 128 (lanes along a row of pixels), or,
+  // channels last, slots t / 4 + 128 u, group t % 4 (four lanes read a pixel's 128 contiguous bytes).
+  int n0, oy0, nl, oyl, ox0;
+  pixel(q0, n0, oy0, ox0);
+  pixel(min(q0 + BQ, ph.Q) - 1, nl, oyl, ox0);
+  const int slots = ((nl - n0) * SH + oyl - oy0 + ph.KH) * SW;  // at most NS: the host checks the worst tile
+  uint32_t voff[NU];  // byte offset of each item at channel 0
+  const int s0 = MODE == kNhwc ? t >> 2 : t % (NT / 4), g = MODE == kNhwc ? t & 3 : t / (NT / 4);
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    const int s = s0 + NT / 4 * u;
+    const int sr = (int)fdiv((uint32_t)s, ph.div_sw), sx = s - sr * SW, row = sr + oy0;
+    const int nn = (int)fdiv((uint32_t)row, ph.div_sh), n = n0 + nn, iy = row - nn * SH - ph.PH, ix = sx - ph.PW;
+    const bool ok = (s < slots) & ((unsigned)iy < (unsigned)H) & ((unsigned)ix < (unsigned)W);
+    voff[u] = !ok ? kOOB
+              : MODE == kNhwc ? (uint32_t)(((n * H + iy) * W + ix) * C * 4 + 32 * g)
+                              : (uint32_t)((n * C * HW + iy * W + ix) * 4 + 8 * g * HW * 4);
+  }
+  float rb[NU][8];
+  auto gload = [&](int cb) {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      if constexpr (MODE == kNhwc) {
+        const float4 f0 = bload4(xr, voff[u], (uint32_t)(cb * 128)), f1 = bload4(xr, voff[u], (uint32_t)(cb * 128 + 16));
+        float* const d = rb[u];
+        d[0] = f0.x, d[1] = f0.y, d[2] = f0.z, d[3] = f0.w, d[4] = f1.x, d[5] = f1.y, d[6] = f1.z, d[7] = f1.w;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) rb[u][e] = bload(xr, voff[u], (uint32_t)((cb * 32 + e) * HW * 4));
+      }
+    }
+  };
+  auto sstore = [&]() {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      uint32_t h[4], m[4], l[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) split_bf16(rb[u][2 * e], rb[u][2 * e + 1], h[e], m[e], l[e]);
+      if (s0 + NT / 4 * u < slots) {
+        uint4* const o = Bs + g * NS + s0 + NT / 4 * u;
+        o[0] = make_uint4(h[0], h[1], h[2], h[3]);
+        o[4 * NS] = make_uint4(m[0], m[1], m[2], m[3]);
+        o[8 * NS] = make_uint4(l[0], l[1], l[2], l[3]);
+      }
+    }
+  };
+
+  // The filter's K-block of tap and channel block cb, 1 KB per instruction.
+  const omt_u32x4 wr = rsrc_words(a.wsplit, a.wsplit_bytes);
+  constexpr int AKB = BP * 12 / 64;
+  const uint32_t alds = lds_addr(reinterpret_cast<const float*>(lds));
+  const int ncb = ph.K > 0 ? C / BK : 0;  // a phase that no tap reaches writes zeros
+  auto aload = [&](int tap0, int cb, int buf) {  // taps tap0 .. tap0 + AT - 1, those that exist
+#pragma unroll
+    for (int v = 0; v < AT; ++v) {
+      if (tap0 + v >= KK) break;
+      const uint32_t src = (uint32_t)((ph.soff + (tile.y * ph.snkb + (tap0 + v) * (C / BK) + cb) * ATAP) * 16);
+#pragma unroll
+      for (int i = 0; i < (AKB + NW - 1) / NW; ++i) {
+        const int c = wave + NW * i;
+        if (AKB % NW == 0 || c < AKB)
+          lds_load_b128s(wr, alds + (uint32_t)((buf * ABUF + v * ATAP) * 16 + c * 1024), (uint32_t)(lane * 16),
+                         src + (uint32_t)(c * 1024));
+      }
+    }
+  };
+  // End of a step: this wave's LDS writes and its filter loads done. GL: the source loads issued after the filter's.
+  auto sync = [&](auto gl) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(decltype(gl)::value) & ~0xF00);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  using Done = std::integral_constant<int, 0>;
+  using Loading = std::integral_constant<int, MODE == kNhwc ? 2 * NU : 8 * NU>;
+
+  // The slot of each of this lane's columns at tap (0, 0); columns past Q read slot 0 (their sums are not stored).
+  const int la = wp * WP + (lane & 15), grp = lane >> 4;
+  int sb[TJ];
+#pragma unroll
+  for (int j = 0; j < TJ; ++j) {
+    const int q = q0 + wq * WQ + 16 * j + (lane & 15);
+    int n, oy, x;
+    pixel(min(q, ph.Q - 1), n, oy, x);
+    sb[j] = grp * NS + (q < ph.Q ? ((n - n0) * SH + oy - oy0) * SW + x : 0);
+  }
+
+  omt_f32x4 acc[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[i][j] = omt_f32x4{0.f, 0.f, 0.f, 0.f};
+  // x's fragments one column tile ahead where the registers allow it (a spilled load is waited for at once)
+  constexpr int NBV = TI >= 4 ? 1 : 2;
+  omt_bf16x8 av[3][TI], bv[NBV][3];
   omt_f32x4 s[2][TI];  // the K-block's sums of column tiles j and j - 1
 #pragma unroll
   for (int i = 0; i < TI; ++i) s[(TJ - 1) & 1][i] = omt_f32x4{0.f, 0.f, 0.f, 0.f};
-  auto step = [&](int it, auto setc) {
-    constexpr int S = decltype(setc)::value;  // it & 1
+  auto mfma_block = [&](int abase, int tslot) {  // one tap's K-block
     constexpr int za[6] = {2, 0, 1, 1, 0, 0}, zb[6] = {0, 2, 1, 0, 1, 0};  // smallest partial products first
-    const auto frag = [&](int unit) { return __builtin_bit_cast(omt_bf16x8, lds[S * BUF + unit]); };
-    const auto bread = [&](int j, int z) { return frag(12 * BP + (4 * z + grp) * BS + lb + 16 * j); };
+    const auto bread = [&](int j, int z) { return __builtin_bit_cast(omt_bf16x8, Bs[4 * z * NS + sb[j] + tslot]); };
 #pragma unroll
     for (int z = 0; z < 3; ++z) {
 #pragma unroll
-      for (int i = 0; i < TI; ++i) av[za[z]][i] = frag((4 * za[z] + grp) * BP + la + 16 * i);
+      for (int i = 0; i < TI; ++i)
+        av[za[z]][i] = __builtin_bit_cast(omt_bf16x8, lds[abase + (4 * za[z] + grp) * BP + la + 16 * i]);
       bv[0][zb[z]] = bread(0, zb[z]);
     }
-    aload(it + 1, S ^ 1);
-    gload(kbeg + (it + 2) * BK, S);
-    // Column tile j's MFMAs run beside the additions and a quarter of the staging of the tile before.
 #pragma unroll
     for (int j = 0; j < TJ; ++j) {
 #pragma unroll
-      for (int z = 0; z < 3; ++z)
-        if (j + 1 < TJ) bv[(j + 1) & 1][zb[z]] = bread(j + 1, zb[z]);
+      for (int z = 0; z < 3; ++z) {
+        if (NBV == 2 && j + 1 < TJ) bv[(j + 1) % NBV][zb[z]] = bread(j + 1, zb[z]);
+        if (NBV == 1 && j > 0) bv[0][zb[z]] = bread(j, zb[z]);
+      }
 #pragma unroll
       for (int i = 0; i < TI; ++i) s[j & 1][i] = omt_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int z = 0; z < 6; ++z)
 #pragma unroll
         for (int i = 0; i < TI; ++i)
-          s[j & 1][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[za[z]][i], bv[j & 1][zb[z]], s[j & 1][i], 0, 0, 0);
-      if (j > 0) sstore(j - 1, S ^ 1, S ^ 1);
-      if (j == TJ - 1) sstore(j, S ^ 1, S ^ 1);
+          s[j & 1][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[za[z]][i], bv[j % NBV][zb[z]], s[j & 1][i], 0, 0, 0);
 #pragma unroll
       for (int i = 0; i < TI; ++i) acc[i][(j + TJ - 1) % TJ] += s[(j + 1) & 1][i];
       __builtin_amdgcn_sched_barrier(0);
     }
-    sync();
   };
-  // Whole pairs of steps in the loop and an odd last one after it: a conditional second step merges two load histories
-  // at the loop head, where the compiler then waits for every load in flight.
-  int it = 0;
-  for (; it + 1 < nk; it += 2) {
-    step(it, std::integral_constant<int, 0>{});
-    step(it + 1, std::integral_constant<int, 1>{});
+
+  if (ncb > 0) {
+    gload(0);
+    aload(0, 0, 0);
+    sstore();
   }
-  if (it < nk) step(it, std::integral_constant<int, 0>{});
+  sync(Done{});
+  int buf = 0;
+  for (int cb = 0; cb < ncb; ++cb) {
+    const bool more = cb + 1 < ncb;
+    int ky = 0, kx = 0;
+    for (int tap = 0; tap < KK; tap += AT, buf ^= 1) {
+      const bool last = tap + AT >= KK;
+      if (!last || more) aload(last ? 0 : tap + AT, last ? cb + 1 : cb, buf ^ 1);
+      const bool load = tap == 0 && more;
+      if (load) gload(cb + 1);  // the next channels, in flight through this step and the next
+#pragma unroll
+      for (int v = 0; v < AT; ++v) {
+        if (tap + v >= KK) break;
+        mfma_block(buf * ABUF + v * ATAP, ky * SW + kx);
+        const bool wrap = ++kx == KW;
+        kx = wrap ? 0 : kx;
+        ky += wrap;
+      }
+      if (load && !last) sync(Loading{});
+      else sync(Done{});
+    }
+    if (more) {
+      sstore();
+      sync(Done{});
+    }
+  }
 #pragma unroll
   for (int i = 0; i < TI; ++i) acc[i][TJ - 1] += s[(TJ - 1) & 1][i];
 
-  static_assert(NW * row_epi_floats<WQ>() <= 4 * BUF && gather_lds_floats<64, 128, 16>() <= 4 * BUF,
-                "epilogue and fp32 tile fit the LDS");
+  static_assert(NW * row_epi_floats<WQ>() <= 4 * 12 * NS && gather_lds_floats<64, 128, 16>() <= 4 * 12 * NS, "LDS");
   float* const fl = reinterpret_cast<float*>(lds);
-  if (split_redo<TI, TJ, NW>(acc, wave, lane, reinterpret_cast<uint32_t*>(lds))) {
-    // the fp32 tile is the work of four waves; a barrier waits for the waves that have not ended
-    if (wave >= 4) return;
-    constexpr int FQ = BQ / 128, FP = BP / 64, FMODE = MODE == kTapMajor ? kTapInPlace : MODE;
-#pragma unroll 1
-    for (int f = 0; f < FP * FQ; ++f) {
-      gather_tile<64, 128, 32, 64, 16, FMODE, false, 2>(a, bx * FQ + f % FQ, by * FP + f / FQ, bz, fl);
-      __syncthreads();
-    }
-    return;
-  }
-  if constexpr (MODE == kNhwc)
-    gather_epilogue_nhwc<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane, zs);
-  else if (a.d2s && !a.part)
-    d2s_epilogue<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane);
-  else if (a.rows)
-    row_epilogue<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane, fl + wave * row_epi_floats<WQ>());
+  if (split_redo<TI, TJ, NW>(acc, wave, lane, reinterpret_cast<uint32_t*>(lds)))
+    split_redo_tiles<BP, BQ, MODE>(a, ntiles, wave, fl);
   else
-    gather_epilogue<TI, TJ, WP, WQ>(a, ph, acc, q0, p0, wp, wq, lane, zs);
+    split_epilogue<BP, BQ, WP, WQ, MODE>(a, ph, acc, tile.x, tile.y, 0, wave, lane, fl);
 }
 
-template <int BP, int BQ, int WP, int WQ, int MODE>
-__global__ void __launch_bounds__(kSplitNT, 2) conv_gather_split_kernel(const GatherArgs a) {
-  __shared__ __attribute__((aligned(16))) uint4 lds[2 * split_lds_units<BP, BQ, MODE>()];
-  const TileId t = xcd_block_tile(kTileGroup);
-  gather_split_tile<BP, BQ, WP, WQ, MODE>(a, t.x, t.y, t.z, lds);
+template <int BP, int WP, int MODE>
+__global__ void __launch_bounds__(kSplitNT, 2) conv_gather_window_kernel(const GatherArgs a, const int ntiles) {
+  __shared__ __attribute__((aligned(16))) uint4 lds[2 * 12 * 128 + 12 * kWindowSlots];
+  gather_window_tile<BP, WP, MODE>(a, ntiles, lds);
 }
 
 // 1x1, stride 1, unpadded convolutions (and their grad input, a 1x1 convolution with the transposed filter) with a
@@ -2706,13 +2994,43 @@ static void gather_dl_dispatch(int ti, const GatherArgs& a, dim3 grid, hipStream
   }
 }
 
+// Whether a split launch runs the window tile: unsplit, stride 1, whole blocks of 32 channels, more than one tap, and
+// the input rows under any 256 consecutive output pixels of every phase fit its LDS.
+static bool window_ok(const GatherArgs& a) {
+  if (a.part || a.C % 32 != 0) return false;
+  int64_t taps = 0;
+  for (int f = 0; f < a.nphase; ++f) {
+    const Phase& p = a.ph[f];
+    if (p.S != 1) return false;
+    taps += p.KH * p.KW;
+    const int64_t rows = (kSplitBQ - 1 + p.OW - 1) / p.OW + 1, images = (rows - 1 + p.OH - 1) / p.OH + 1;
+    if ((rows + images * (p.KH - 1)) * (p.OW + p.KW - 1) > kWindowSlots)
+      return false;
+  }
+  return taps > a.nphase;
+}
 // The split tile in its K order: tap-major, channel-major, or over a channels-last source.
 template <int MODE>
 static void gather_split_dispatch(const GatherArgs& a, dim3 grid, hipStream_t s) {
-  if (split_bp(a.P) == 64)
-    hipLaunchKernelGGL((conv_gather_split_kernel<64, 256, 32, 64, MODE>), grid, dim3(kSplitNT), 0, s, a);
+  const int ntiles = (int)(grid.x * grid.y * grid.z);
+  GatherArgs b = a;
+  b.gx = (int)grid.x;
+  b.gy = (int)grid.y;
+  const dim3 g(grid.z == 1 ? (unsigned)std::min<int64_t>(ntiles, kCUs) : (unsigned)ntiles);
+  const bool h64 = split_bp(a.P) == 64;
+  if constexpr (MODE != kGeneric)
+    if (window_ok(a)) {
+      const dim3 one((unsigned)ntiles);
+      if (h64)
+        hipLaunchKernelGGL((conv_gather_window_kernel<64, 32, MODE>), one, dim3(kSplitNT), 0, s, b, ntiles);
+      else
+        hipLaunchKernelGGL((conv_gather_window_kernel<128, 64, MODE>), one, dim3(kSplitNT), 0, s, b, ntiles);
+      return;
+    }
+  if (h64)
+    hipLaunchKernelGGL((conv_gather_split_kernel<64, 256, 32, 64, MODE>), g, dim3(kSplitNT), 0, s, b, ntiles);
   else
-    hipLaunchKernelGGL((conv_gather_split_kernel<128, 256, 64, 64, MODE>), grid, dim3(kSplitNT), 0, s, a);
+    hipLaunchKernelGGL((conv_gather_split_kernel<128, 256, 64, 64, MODE>), g, dim3(kSplitNT), 0, s, b, ntiles);
 }
 // Lays out the phases of the split tile's packed filter (a.ph and a.P set) and returns its bytes.
 static size_t split_layout(GatherArgs& a) {
@@ -2721,6 +3039,8 @@ static size_t split_layout(GatherArgs& a) {
     a.ph[f].soff = (int)units;
     a.ph[f].snkb = (int)std::max<int64_t>(1, cdiv(a.ph[f].K, kSplitBK));
     units += cdiv(a.P, split_bp(a.P)) * a.ph[f].snkb * 12 * split_bp(a.P);
+    a.ph[f].div_sw = make_fastdiv((uint32_t)(a.ph[f].OW + a.ph[f].KW - 1));
+    a.ph[f].div_sh = make_fastdiv((uint32_t)(a.ph[f].OH + a.ph[f].KH - 1));
   }
   return (size_t)units * 16;
 }

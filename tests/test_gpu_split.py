@@ -36,6 +36,13 @@ SHAPES = [
     (1, 16, 64, 15, 17, 3, 1, 1), (1, 48, 65, 16, 16, 3, 1, 1), (2, 32, 128, 11, 12, 1, 1, 0),
     (1, 64, 129, 257, 1, 1, 1, 0), (3, 33, 63, 9, 11, 3, 1, 1), (2, 7, 200, 10, 13, 5, 2, 2),
     (2, 80, 48, 12, 9, 3, 2, 1), (2, 128, 16, 7, 7, 3, 1, 1), (1, 3, 64, 33, 29, 7, 2, 3), (40, 17, 31, 1, 1, 1, 1, 0),
+    # more tiles than CUs, so that a workgroup runs several, of one K-block and of three
+    (2, 16, 64, 190, 190, 1, 1, 0), (2, 72, 40, 190, 183, 1, 1, 0),
+    # window tiles (channels % 32): tiles over several images, windows of 5 and 2 rows, strided phases (grad input),
+    # the super-pixel grad input, the widest rows that fit (64: 594 of 596 slots) and rows that do not
+    (9, 32, 70, 7, 7, 3, 1, 1), (3, 64, 130, 14, 9, 3, 1, 1), (2, 96, 64, 20, 11, 5, 1, 2), (2, 32, 32, 9, 9, 2, 1, 0),
+    (3, 32, 64, 17, 15, 3, 2, 1), (2, 3, 64, 33, 29, 11, 4, 2), (2, 32, 33, 64, 64, 3, 1, 1), (1, 32, 16, 5, 200, 3, 1, 1),
+    (2, 64, 64, 5, 3, 3, 1, 3),
 ]
 
 
@@ -61,13 +68,14 @@ def test_split_tile_is_as_exact_as_the_fp32_tile(cuda, ops, shape):
         ops.clear_conv_plans()
 
 
+@pytest.mark.parametrize("ci", [48, 64], ids=["split", "window"])
 @pytest.mark.parametrize("kind", ["inf", "nan", "huge", "tiny", "overflow"])
-def test_split_tile_falls_back_on_values_it_cannot_split(cuda, ops, kind):
+def test_split_tile_falls_back_on_values_it_cannot_split(cuda, ops, kind, ci):
     """Infinities, NaN, values that round past the largest bf16, sums that overflow, and inputs whose low terms
     underflow: the tile is computed again in fp32, so every output is the fp32 tile's to the bit where the whole tile
     is affected, and equal in kind (NaN, infinity, finite within rounding) elsewhere."""
     rng = np.random.default_rng(3)
-    n, ci, co, h = 2, 48, 96, 13
+    n, co, h = 2, 96, 13
     x, wt = rnd(rng, n, ci, h, h), rnd(rng, co, ci, 3, 3, scale=0.05)
     if kind in ("inf", "nan"):
         x[1, 5, 6, 7] = np.inf if kind == "inf" else np.nan
@@ -93,10 +101,26 @@ def test_split_tile_falls_back_on_values_it_cannot_split(cuda, ops, kind):
                 assert np.array_equal(a[f], b[f])
             else:
                 scale = np.abs(b[f]).max() if kind == "huge" else np.sqrt((b[f].astype(np.float64) ** 2).mean())
-                # both within K 2^-24 relative of the exact sums (K = 432 products)
-                assert np.abs(a[f].astype(np.float64) - b[f]).max() <= 2 * 432 * 2.0 ** -24 * scale
+                # both within K 2^-24 relative of the exact sums (K = 9 ci products)
+                assert np.abs(a[f].astype(np.float64) - b[f]).max() <= 2 * 9 * ci * 2.0 ** -24 * scale
     finally:
         ops.clear_conv_plans()
+
+
+def test_a_workgroup_redoes_all_its_tiles(cuda, ops):
+    """283 tiles on 256 CUs: a NaN in one of them has its workgroup compute all its tiles again in fp32."""
+    rng = np.random.default_rng(11)
+    x, wt = rnd(rng, 2, 16, 190, 190), rnd(rng, 64, 16, 1, 1)
+    x[0, 3, 1, 2], x[1, 7, 189, 189] = np.nan, np.inf
+    t = [torch.from_numpy(a).to(cuda) for a in (x, wt)]
+    try:
+        a = run(ops, "fwd", t, x, wt, None, 1, 0, SPLIT)
+        b = run(ops, "fwd", t, x, wt, None, 1, 0, FP32)
+    finally:
+        ops.clear_conv_plans()
+    assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b))
+    f = np.isfinite(b)  # both within K 2^-24 relative of the exact sums of up to K = 16 products of a few units each
+    assert np.abs(a[f].astype(np.float64) - b[f]).max() <= 2 * 16 * 2.0 ** -24 * np.abs(b[f]).max()
 
 
 WSPLIT, WSPLIT_NHWC, WFP32 = 4, 3, 2  # grad-weight tiles

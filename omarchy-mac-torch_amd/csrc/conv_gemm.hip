@@ -76,7 +76,6 @@ struct Phase {
   int woff;               // offset of this phase's [P][K] weights (floats)
   int ky0, kx0;           // grad input read straight from w: the phase's first filter tap
   int soff, snkb;         // split tile: the phase's first 16-byte unit of the packed filter, and its K-blocks
-  FastDiv div_sw, div_sh; // window tile: OW + KW - 1 (a row of staged pixels), OH + KH - 1 (an image's rows of them)
   FastDiv div_ohw, div_ow, div_kk, div_kw;
 };
 
@@ -1172,13 +1171,19 @@ __device__ __forceinline__ void gather_window_tile(const GatherArgs& a, const in
   pixel(q0, n0, oy0, ox0);
   pixel(min(q0 + BQ, ph.Q) - 1, nl, oyl, ox0);
   const int slots = ((nl - n0) * SH + oyl - oy0 + ph.KH) * SW;  // at most NS: the host checks the worst tile
+  // v / d for 0 <= v < 2^31 and a quotient below 2^20, where v times d's rounded reciprocal is off by less than one
+  const float rsw = 1.f / (float)SW, rsh = 1.f / (float)SH;
+  const auto quotient = [](int v, int d, float rd) {
+    const int q = (int)((float)v * rd), r = v - q * d;
+    return q + (r >= d) - (r < 0);
+  };
   uint32_t voff[NU];  // byte offset of each item at channel 0
   const int s0 = MODE == kNhwc ? t >> 2 : t % (NT / 4), g = MODE == kNhwc ? t & 3 : t / (NT / 4);
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
     const int s = s0 + NT / 4 * u;
-    const int sr = (int)fdiv((uint32_t)s, ph.div_sw), sx = s - sr * SW, row = sr + oy0;
-    const int nn = (int)fdiv((uint32_t)row, ph.div_sh), n = n0 + nn, iy = row - nn * SH - ph.PH, ix = sx - ph.PW;
+    const int sr = quotient(s, SW, rsw), sx = s - sr * SW, row = sr + oy0;
+    const int nn = quotient(row, SH, rsh), n = n0 + nn, iy = row - nn * SH - ph.PH, ix = sx - ph.PW;
     const bool ok = (s < slots) & ((unsigned)iy < (unsigned)H) & ((unsigned)ix < (unsigned)W);
     voff[u] = !ok ? kOOB
               : MODE == kNhwc ? (uint32_t)(((n * H + iy) * W + ix) * C * 4 + 32 * g)
@@ -3039,8 +3044,6 @@ static size_t split_layout(GatherArgs& a) {
     a.ph[f].soff = (int)units;
     a.ph[f].snkb = (int)std::max<int64_t>(1, cdiv(a.ph[f].K, kSplitBK));
     units += cdiv(a.P, split_bp(a.P)) * a.ph[f].snkb * 12 * split_bp(a.P);
-    a.ph[f].div_sw = make_fastdiv((uint32_t)(a.ph[f].OW + a.ph[f].KW - 1));
-    a.ph[f].div_sh = make_fastdiv((uint32_t)(a.ph[f].OH + a.ph[f].KH - 1));
   }
   return (size_t)units * 16;
 }

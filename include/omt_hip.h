@@ -61,9 +61,10 @@ enum {
   OMT_DIR_WGRAD_NHWC = 5
 };
 
-/* A dense convolution's launch plan: tile index (into the direction's tile table, omt_conv_num_tiles) and number of
- * K slices (split K; rounded to whole K-blocks per slice). Replaces ConvPlan's tile and split-K multiplier
- * (csrc/omt.h:230-236). */
+/* A dense convolution's launch plan: tile index (into the direction's table of fp32 tiles, omt_conv_num_tiles, or
+ * OMT_TILE_SPLIT) and number of K slices (split K; rounded to whole K-blocks per slice). Replaces ConvPlan's tile and
+ * split-K multiplier (csrc/omt.h:230-236). */
+#define OMT_TILE_SPLIT 256 /* the tile that computes fp32 products on the bf16 matrix cores: forward and grad input */
 typedef struct omt_conv_plan {
   int32_t tile, slices;
 } omt_conv_plan;
@@ -239,7 +240,7 @@ int omt_slice_sums(const omt_slice_sum* sums, int count, void* stream);
  * grad weight needs co % 4 == 0 (else OMT_UNSUPPORTED). A forward of ci % 16 != 0 (the 3-channel stem) and a grad
  * input of co % 16 != 0 gather element by element on one fixed plan, a grad weight of ci % 4 != 0 loads its columns
  * one by one: same LDS staging and MFMA order; those gathers are not tuned. Plans: directions OMT_DIR_FWD_NHWC,
- * OMT_DIR_DGRAD_NHWC, OMT_DIR_WGRAD_NHWC (tile indices below omt_conv_num_tiles of the direction). Bias and ReLU
+ * OMT_DIR_DGRAD_NHWC, OMT_DIR_WGRAD_NHWC (tile indices as in omt_conv_plan). Bias and ReLU
  * epilogue bits as in omt_conv_fwd; no BN loader. */
 size_t omt_conv_fwd_nhwc_workspace(const omt_conv_geo* g);
 int omt_conv_fwd_nhwc(const omt_conv_geo* g, const float* x, const float* w, const float* bias, unsigned epilogue,
@@ -256,8 +257,8 @@ int omt_conv_wgrad_nhwc(const omt_conv_geo* g, const float* x, const float* gy, 
  * Every dense-conv call and workspace query resolves its plan from a process-wide cache keyed by (direction,
  * geometry); without an entry a cost model picks it. Changing an entry between a workspace query and the launch it
  * sized can make the launch fail with OMT_INVALID (workspace too small), never overrun the workspace.
- * omt_conv_autotune times the candidates (every tile of the first max_tiles, <= 0 meaning all, times a few K
- * splits) on scratch buffers, each as replays of a captured HIP graph of several calls on a private stream ordered
+ * omt_conv_autotune times the candidates (every tile of the first max_tiles, <= 0 meaning all, and with all of them
+ * the split tile on layers of 2^30 multiply-adds or more, times a few K splits) on scratch buffers, each as replays of a captured HIP graph of several calls on a private stream ordered
  * after `stream` (so a plan's extra launches cost what they cost in a replayed step), stores the fastest in the cache
  * and returns it in *best (may be NULL). It synchronizes `stream`, allocates through omt_malloc, and refuses
  * (OMT_UNSUPPORTED) while `stream` is capturing. The cache is in key order for omt_conv_plan_entry (i < omt_conv_plan_count()). */

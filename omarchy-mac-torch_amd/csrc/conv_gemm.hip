@@ -2879,7 +2879,7 @@ static int pick_tile(const Tile (&tiles)[N], int64_t P, int64_t Q, int64_t z, in
 // 64x64 input: 64 channels over 8192 pixels) twice the workgroups of the 64 x 64 tile, so that every CU holds one
 // without a K split.
 static const Tile kGatherTiles[] = {
-    {64, 256, 64, 64, 1.00f},     {128, 256, 64, 64, 2.00f, 32, 0, 1}, {64, 128, 32, 64, 0.92f},
+    {64, 256, 64, 64, 1.00f},     {128, 128, 64, 64, 1.00f},    {64, 128, 32, 64, 0.92f},
     {32, 256, 32, 64, 0.90f},     {16, 256, 16, 64, 0.80f},     {64, 64, 32, 32, 0.80f},
     {64, 64, 32, 32, 0.90f, 64},  {64, 128, 32, 64, 0.95f, 32}, {128, 64, 64, 32, 0.95f, 32},
     {64, 64, 32, 32, 0.85f, 16, 4}, {64, 128, 32, 64, 0.95f, 16, 3}, {64, 64, 32, 32, 0.90f, 32, 3},
@@ -2894,6 +2894,11 @@ static const Tile kGatherTiles[] = {
 // load), on tiles whose filter tile has whole runs per thread (BP BK >= 1024) and that are not the 1x1 streaming
 // tile; elsewhere it runs as the first variant.
 constexpr int kNGather = (int)(sizeof(kGatherTiles) / sizeof(kGatherTiles[0]));
+// The split-bf16 tile (bp by the output channels: tile_bp) is plan tile OMT_TILE_SPLIT, beside the table, whose indices
+// stay those of the fp32 tiles in every plan that a program keeps: tap-major where C is a multiple of its runs, else
+// channel-major.
+static const Tile kSplitTile = {128, 256, 64, 64, 2.00f, 32, 0, 1};
+static_assert(OMT_TILE_SPLIT >= 3 * kNGather, "the split tile's index");
 constexpr int kStreamTile = 13;
 // The filter-stationary tiles 17-19 (conv1x1_wst_kernel): 64 TJ output channels per workgroup at K 64 (TJ 4, 2, 2),
 // half as many at K 128 (the same filter registers), pixel tiles of 32, 32 and 64; their resident workgroups per CU
@@ -2901,7 +2906,7 @@ constexpr int kStreamTile = 13;
 constexpr int kWstFirst = 17;
 constexpr int kWstOcc[3][2] = {{2, 3}, {4, 3}, {2, 1}};  // as registers and LDS (input + staging) allow
 static int wst_shape(int t) { return t % kNGather - kWstFirst; }  // conv1x1_stream_kernel; tile 17 (conv1x1_wst_kernel) runs as it where it does not apply
-static const Tile& gtile(int t) { return kGatherTiles[t % kNGather]; }
+static const Tile& gtile(int t) { return t == OMT_TILE_SPLIT ? kSplitTile : kGatherTiles[t % kNGather]; }
 static bool gcm(int t) { return t >= kNGather && t < 2 * kNGather; }
 static bool wplace_tile(int t) {
   const Tile& tl = gtile(t);
@@ -2958,6 +2963,7 @@ template <int MODE, bool BN>
 static void gather_dispatch(int ti, const GatherArgs& a, dim3 grid, hipStream_t s) {
   switch (ti) {
     case 0: hipLaunchKernelGGL((conv_gather_kernel<64, 256, 64, 64, 16, MODE, BN, BN ? 1 : 2>), grid, dim3(256), 0, s, a); break;
+    case 1: hipLaunchKernelGGL((conv_gather_kernel<128, 128, 64, 64, 16, MODE, BN, 2>), grid, dim3(256), 0, s, a); break;
     case 2: hipLaunchKernelGGL((conv_gather_kernel<64, 128, 32, 64, 16, MODE, BN, 2>), grid, dim3(256), 0, s, a); break;
     case 3: hipLaunchKernelGGL((conv_gather_kernel<32, 256, 32, 64, 16, MODE, BN, 2>), grid, dim3(256), 0, s, a); break;
     case 4: hipLaunchKernelGGL((conv_gather_kernel<16, 256, 16, 64, 16, MODE, BN, 2>), grid, dim3(256), 0, s, a); break;
@@ -2981,6 +2987,7 @@ static void gather_inplace_dispatch(int ti, const GatherArgs& a, dim3 grid, hipS
   constexpr int M = kTapInPlace;
   switch (ti) {
     case 0: hipLaunchKernelGGL((conv_gather_kernel<64, 256, 64, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
+    case 1: hipLaunchKernelGGL((conv_gather_kernel<128, 128, 64, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
     case 6: hipLaunchKernelGGL((conv_gather_kernel<64, 64, 32, 32, 64, M, false, 2>), grid, dim3(256), 0, s, a); break;
     case 8: hipLaunchKernelGGL((conv_gather_kernel<128, 64, 64, 32, 32, M, false, 2>), grid, dim3(256), 0, s, a); break;
     case 2: case 10: hipLaunchKernelGGL((conv_gather_kernel<64, 128, 32, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
@@ -3066,6 +3073,7 @@ static void gather_nhwc_dispatch(int ti, const GatherArgs& a, dim3 grid, hipStre
   constexpr int M = kNhwc;
   switch (ti) {
     case 0: hipLaunchKernelGGL((conv_gather_kernel<64, 256, 64, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
+    case 1: hipLaunchKernelGGL((conv_gather_kernel<128, 128, 64, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
     case 2: hipLaunchKernelGGL((conv_gather_kernel<64, 128, 32, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
     case 3: hipLaunchKernelGGL((conv_gather_kernel<32, 256, 32, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
     case 4: hipLaunchKernelGGL((conv_gather_kernel<16, 256, 16, 64, 16, M, false, 2>), grid, dim3(256), 0, s, a); break;
@@ -3094,9 +3102,11 @@ static const int kSliceChoices[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
 // - a split pays the partial round trip through HBM (~1.7 KB/clock) and one more launch (~7000 clocks).
 // `fixed` (a tuned or requested plan) replaces the estimate: its slice count is rounded to whole K-blocks per slice.
 // nhwc_c > 0: a channels-last gather over nhwc_c source channels, which runs the staged tiles 0 .. kNhwcTiles - 1 whose
-// K-block divides nhwc_c (a fixed plan outside them runs as tile kNhwcDefault).
+// K-block (the split tile, whose run) divides nhwc_c (a fixed plan outside them runs as tile kNhwcDefault).
 constexpr int kNhwcTiles = 9, kNhwcDefault = 5;
-static bool nhwc_tile_ok(int t, int64_t c) { return t >= 0 && t < kNhwcTiles && c % kGatherTiles[t].run() == 0; }
+static bool nhwc_tile_ok(int t, int64_t c) {
+  return ((t >= 0 && t < kNhwcTiles) || t == OMT_TILE_SPLIT) && c % gtile(t).run() == 0;
+}
 static GatherPlan gather_plan(int64_t P, int64_t Q, int64_t K, int64_t z, const omt_conv_plan* fixed,
                               int64_t nhwc_c = 0) {
   const int64_t kk = K > 0 ? K : 1;
@@ -3109,8 +3119,9 @@ static GatherPlan gather_plan(int64_t P, int64_t Q, int64_t K, int64_t z, const 
   }
   GatherPlan best{nhwc_c ? kNhwcDefault : 0, 1, cdiv(kk, 16) * 16};
   double best_cost = 1e300;
-  for (int ti = 0; ti < kNGather; ++ti) {
-    const Tile& tl = kGatherTiles[ti];
+  for (int i = 0; i <= kNGather; ++i) {
+    const int ti = i < kNGather ? i : OMT_TILE_SPLIT;
+    const Tile& tl = gtile(ti);
     if (tl.stream) continue;  // chosen by tuning only
     if (nhwc_c && !nhwc_tile_ok(ti, nhwc_c)) continue;
     if (tl.split && !split_pays(P, Q, kk, z)) continue;
@@ -3186,7 +3197,7 @@ static bool wst_ok(const GatherArgs& a, const GatherPlan& pl) {
 }
 // The split tile has no BN loader: its plans run as tile 2 there.
 static GatherPlan eff_plan(const GatherArgs& a, GatherPlan pl) {
-  if (gtile(pl.tile).split && a.bn_mean) pl.tile = pl.tile - pl.tile % kNGather + 2;
+  if (gtile(pl.tile).split && a.bn_mean) pl.tile = 2;
   if (gtile(pl.tile).stream == 2 && !wst_ok(a, pl)) pl.tile = pl.tile - pl.tile % kNGather + kStreamTile;
   if (gtile(pl.tile).stream && !stream_ok(a, pl)) pl.tile = pl.tile - pl.tile % kNGather + 2;
   return pl;
@@ -3439,9 +3450,13 @@ static bool cached_plan(int dir, const omt_conv_geo* g, omt_conv_plan* p) {
   return true;
 }
 static bool wgrad_dir(int dir) { return dir == OMT_DIR_WGRAD || dir == OMT_DIR_WGRAD_NHWC; }
+// The fp32 tiles of a direction.
 static int num_tiles(int dir) {
   if (wgrad_dir(dir)) return dir == OMT_DIR_WGRAD_NHWC ? kWgradSplitNhwc + 1 : kWgradSplit + 1;
   return dir == OMT_DIR_FWD_NHWC || dir == OMT_DIR_DGRAD_NHWC ? kNhwcTiles : 3 * kNGather;
+}
+static bool tile_index_ok(int dir, int t) {
+  return (t >= 0 && t < num_tiles(dir)) || (t == OMT_TILE_SPLIT && !wgrad_dir(dir));
 }
 
 }  // namespace omt
@@ -3507,7 +3522,7 @@ static int conv_fwd_one(const omt_conv_geo* g, const float* x, const float* w, c
     if (int st = launch_check("pack_tapmajor_kernel")) return st;
     a.w = (const float*)workspace;
   }
-  if (!bn && (split ? !gcm(pl.tile) : g->ks > 1 && wplace_tile(pl.tile)) &&
+  if (!bn && (split || (g->ks > 1 && wplace_tile(pl.tile))) &&
       gather_tap_major(g->ci, false, gtile(pl.tile).run())) {
     a.wplace = 1;  // A[co][(ky, kx, ci)] = w[co][ci][ky][kx]
     a.ks = (int)g->ks;
@@ -3829,7 +3844,7 @@ static int dgrad_prepare(const omt_conv_geo* g, const float* gy, const float* w,
     a.w_bytes = (uint32_t)(g->co * g->ci * g->ks * g->ks * 4);
     a.ks = (int)g->ks;
     a.s = (int)g->stride;
-    if ((split ? !gcm(pl.tile) : wplace_tile(pl.tile)) && gather_tap_major(g->co, false, gtile(pl.tile).run())) {
+    if ((split || wplace_tile(pl.tile)) && gather_tap_major(g->co, false, gtile(pl.tile).run())) {
       a.wplace = 2;  // A[ci][(a', b', co)] = w[co][ci][ky0 + s (KH - 1 - a')][kx0 + s (KW - 1 - b')]
       a.w_rowst = (uint32_t)(g->ks * g->ks * 4);
       a.w_cst = (uint32_t)(g->ci * g->ks * g->ks * 4);
@@ -4568,7 +4583,7 @@ OMT_EXPORT int omt_conv_set_plan(int dir, const omt_conv_geo* g, const omt_conv_
     g_plans.erase(key_of(dir, g));
     return OMT_OK;
   }
-  if (plan->tile < 0 || plan->tile >= num_tiles(dir) || plan->slices < 1 || plan->slices > 4096)
+  if (!tile_index_ok(dir, plan->tile) || plan->slices < 1 || plan->slices > 4096)
     return fail(OMT_INVALID, "omt_conv_set_plan: tile %d (of %d) / slices %d out of range", plan->tile, num_tiles(dir),
                 plan->slices);
   g_plans[key_of(dir, g)] = *plan;
@@ -4646,11 +4661,13 @@ std::vector<omt_conv_plan> tune_candidates(int dir, const omt_conv_geo* g, int n
   // (C a multiple of the K-block), no super-pixel grad input, a filter larger than 1x1 in the forward
   const int64_t gather_c = fwd ? g->ci : g->co;
   const bool packs = !(dir == OMT_DIR_FWD && g->ks == 1) && !(dir == OMT_DIR_DGRAD && dgrad_d2s(g));
-  for (int t = 0; t < ntile; ++t) {
+  for (int i = 0; i <= ntile; ++i) {  // the first `ntile` tiles and, with all of them, the split tile
+    if (i == ntile && ntile < num_tiles(dir)) break;
+    const int t = i < ntile ? i : OMT_TILE_SPLIT;
     const Tile& tl = gtile(t);
     if (nhwc && !nhwc_tile_ok(t, gather_c)) continue;
-    if (tl.split && (t >= kNGather || !split_pays(P, Q, K, z))) continue;  // its variants differ in K order alone
-    if (t >= 2 * kNGather && !(wplace_tile(t) && packs && gather_tap_major(gather_c, false, tl.run()))) continue;
+    if (tl.split && !split_pays(P, Q, K, z)) continue;
+    if (!tl.split && t >= 2 * kNGather && !(wplace_tile(t) && packs && gather_tap_major(gather_c, false, tl.run()))) continue;
     if (tl.stream) {
       if (stream_geo && t < kNGather && (tl.stream == 1 || K == 64 || K == 128)) out.push_back({t, 1});
       continue;

@@ -16,6 +16,7 @@ OMT_OK, OMT_UNSUPPORTED, OMT_OOM, OMT_DEVICE_ERROR, OMT_INVALID = range(5)
 OMT_CONV_NONE, OMT_CONV_DENSE, OMT_CONV_DW, OMT_CONV_DWG = range(4)
 OMT_EPI_BIAS, OMT_EPI_RELU = 1, 2
 OMT_DIR_FWD, OMT_DIR_DGRAD, OMT_DIR_WGRAD, OMT_DIR_FWD_NHWC, OMT_DIR_DGRAD_NHWC, OMT_DIR_WGRAD_NHWC = range(6)
+TILE_SPLIT = 256  # OMT_TILE_SPLIT
 NOALLOC_SCRATCH_BYTES = 64 << 20  # OMT_NOALLOC_SCRATCH_BYTES
 (OMT_PW_ADD, OMT_PW_MUL, OMT_PW_RELU, OMT_PW_THRESHOLD_BWD, OMT_PW_HARDSWISH, OMT_PW_HARDSWISH_BWD, OMT_PW_HARDSIGMOID,
  OMT_PW_HARDSIGMOID_BWD, OMT_PW_SCALE, OMT_PW_FILL, OMT_PW_ADD_SCALAR) = range(11)

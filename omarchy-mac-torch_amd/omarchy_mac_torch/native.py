@@ -202,7 +202,7 @@ FALLBACKS = _FallbackView()
 # own tiles and a split-K multiplier.
 TUNE_FILE = os.environ.get(
     "OMARCHY_MAC_TORCH_TUNE_FILE",
-    os.path.expanduser(f"~/.cache/omarchy-mac-torch/tuning-gfx950-t{_lib.L.omt_conv_num_tiles(_lib.OMT_DIR_FWD) // 3}r2.json"))
+    os.path.expanduser(f"~/.cache/omarchy-mac-torch/tuning-gfx950-t{_lib.L.omt_conv_num_tiles(_lib.OMT_DIR_FWD) // 3}r3.json"))
 
 
 class TuningStore:

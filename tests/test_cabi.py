@@ -419,3 +419,30 @@ def test_nhwc_plans_and_workspaces_host_side():
         assert L.omt_conv_fwd_nhwc(ctypes.byref(g), None, fake, None, 0, fake, None, 0, None) == _lib.OMT_INVALID
     finally:
         L.omt_conv_clear_plans()
+
+
+def test_the_split_tile_has_an_index_of_its_own():
+    """OMT_TILE_SPLIT stands beside the fp32 tiles' tables: index 1 is the 128 x 128 fp32 tile in each of its variants
+    and channels last (its filter workspace, or none, not the split tile's packed filter), and the split tile is a plan
+    of every direction with 6 bytes per filter element, rows padded to 64 or 128 and K to 32."""
+    from omarchy_mac_torch import _lib
+    L = _lib.L
+    L.omt_conv_clear_plans()
+    g = _lib.conv_geo(2, 32, 40, 8, 8, 3, 1, 1)
+    ng = L.omt_conv_num_tiles(_lib.OMT_DIR_FWD) // 3
+    filt, split = 40 * 32 * 9 * 4, 64 * 32 * 9 * 6  # 40 and 32 rows: both padded to 64
+    try:
+        for d, query, pack, tiles in (
+                (_lib.OMT_DIR_FWD, L.omt_conv_fwd_workspace, (filt, 0, 0, split), (1, 1 + ng, 1 + 2 * ng)),
+                (_lib.OMT_DIR_DGRAD, L.omt_conv_dgrad_workspace, (0, 0, 0, 64 * 384 * 6), (1, 1 + ng, 1 + 2 * ng)),
+                (_lib.OMT_DIR_FWD_NHWC, L.omt_conv_fwd_nhwc_workspace, (0, split), (1,))):
+            for tile, want in zip(tiles + (_lib.TILE_SPLIT,), pack):
+                assert L.omt_conv_set_plan(d, ctypes.byref(g), ctypes.byref(_lib.ConvPlan(tile, 1))) == _lib.OMT_OK
+                p = _lib.ConvPlan()
+                assert L.omt_conv_get_plan(d, ctypes.byref(g), ctypes.byref(p), None) == _lib.OMT_OK
+                assert (p.tile, query(ctypes.byref(g))) == (tile, want), (d, tile)
+        for d in range(6):
+            for tile in (L.omt_conv_num_tiles(d), _lib.TILE_SPLIT - 1, _lib.TILE_SPLIT + 1):
+                assert L.omt_conv_set_plan(d, ctypes.byref(g), ctypes.byref(_lib.ConvPlan(tile, 1))) == _lib.OMT_INVALID
+    finally:
+        L.omt_conv_clear_plans()

@@ -8,7 +8,7 @@ torch = pytest.importorskip("torch")
 from oracle import oracle as orc  # noqa: E402
 
 pytestmark = pytest.mark.gpu
-SPLIT, FP32 = 1, 2  # gather tiles
+SPLIT, FP32 = 256, 2  # gather tiles (OMT_TILE_SPLIT)
 _CL = torch.channels_last
 
 
@@ -64,6 +64,29 @@ def test_split_tile_is_as_exact_as_the_fp32_tile(cuda, ops, shape):
                 e32 = orc.rel_l2(run(ops, d, t, x, wt, gy, s, p, FP32, slices), ref)
                 err = orc.rel_l2(run(ops, d, t, x, wt, gy, s, p, SPLIT, slices), ref)
                 assert err <= max(e32, 2.0 ** -24), (d, slices, err, e32)
+    finally:
+        ops.clear_conv_plans()
+
+
+@pytest.mark.parametrize("shape", [(2, 32, 130, 9, 15, 3, 1, 1), (3, 48, 64, 10, 7, 3, 2, 1), (2, 64, 140, 8, 8, 1, 1, 0)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_tile_1_is_the_fp32_128x128_tile(cuda, ops, shape):
+    """The split tile has its own index: tile 1 sums as the other fp32 tiles of 16-deep K-blocks do, to the bit, in every
+    K order (its three variants) and channels last."""
+    n, ci, co, h, w, ks, s, p = shape
+    ng = ops.conv_num_tiles("fwd") // 3
+    rng = np.random.default_rng(sum(shape))
+    x, wt = rnd(rng, n, ci, h, w), rnd(rng, co, ci, ks, ks)
+    gy = rnd(rng, n, co, (h + 2 * p - ks) // s + 1, (w + 2 * p - ks) // s + 1)
+    t = [torch.from_numpy(a).to(cuda) for a in (x, wt, gy)]
+    tc = [a.contiguous(memory_format=_CL) for a in t]
+    try:
+        for d in ("fwd", "dgrad", "fwd_nhwc", "dgrad_nhwc"):
+            for v in (0, ng, 2 * ng) if d in ("fwd", "dgrad") else (0,):
+                for slices in (1, 3):
+                    u = tc if d.endswith("nhwc") else t
+                    a, b = (run(ops, d, u, x, wt, gy, s, p, tile + v, slices) for tile in (1, 2))
+                    assert np.array_equal(a, b), (d, v, slices)
     finally:
         ops.clear_conv_plans()
 

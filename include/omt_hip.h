@@ -64,7 +64,7 @@ enum {
 /* A dense convolution's launch plan: tile index (into the direction's table of fp32 tiles, omt_conv_num_tiles, or
  * OMT_TILE_SPLIT) and number of K slices (split K; rounded to whole K-blocks per slice). Replaces ConvPlan's tile and
  * split-K multiplier (csrc/omt.h:230-236). */
-#define OMT_TILE_SPLIT 256 /* the tile that computes fp32 products on the bf16 matrix cores: forward and grad input */
+#define OMT_TILE_SPLIT 256 /* the tiles that compute fp32 products on the bf16 matrix cores */
 typedef struct omt_conv_plan {
   int32_t tile, slices;
 } omt_conv_plan;

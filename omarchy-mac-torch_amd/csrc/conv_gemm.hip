@@ -2862,7 +2862,6 @@ static int pick_tile(const Tile (&tiles)[N], int64_t P, int64_t Q, int64_t z, in
   double best_cost = 1e300;
   for (size_t i = 0; i < N; ++i) {
     const Tile& tl = tiles[i];
-    if (tl.split) continue;
     int64_t blocks = cdiv(P, tl.bp) * cdiv(Q, tl.bq) * z;
     int64_t rounds = cdiv(blocks, slots);
     double cost = (double)rounds * tl.bp * tl.bq / tl.eff;
@@ -2930,16 +2929,11 @@ static bool split_pays(int64_t P, int64_t Q, int64_t K, int64_t z) {
 
 static const Tile kWgradTiles[] = {
     {64, 128, 32, 64, 1.00f}, {128, 64, 32, 64, 1.00f}, {64, 64, 32, 32, 0.85f}, {32, 128, 16, 64, 0.85f},
-    {128, 256, 64, 64, 2.00f, 32, 0, 1},
 };
-// The split tile (conv_wgrad_split_kernel, its shape by wgrad_split_shape): the fifth plan of the NCHW directions.
-// Channels last it is the fourth where each run of eight columns is channels of one tap (C % 8 == 0); elsewhere that
-// plan is the fp32 tile of its index.
-constexpr int kWgradSplit = 4, kWgradSplitNhwc = 3;
-static int wgrad_split_tile_of(int dir) { return dir == OMT_DIR_WGRAD_NHWC ? kWgradSplitNhwc : kWgradSplit; }
-static bool wgrad_is_split(int dir, const omt_conv_geo* g, int tile) {
-  return tile == wgrad_split_tile_of(dir) && (dir != OMT_DIR_WGRAD_NHWC || g->ci % 8 == 0);
-}
+constexpr int kNWgrad = (int)(sizeof(kWgradTiles) / sizeof(kWgradTiles[0]));
+// The split tile (conv_wgrad_split_kernel, its shape by wgrad_split_shape) is plan tile OMT_TILE_SPLIT. Channels last it
+// needs each run of eight columns to be channels of one tap (C % 8 == 0); elsewhere that plan runs as tile 2.
+static bool wgrad_split_ok(int dir, const omt_conv_geo* g) { return dir != OMT_DIR_WGRAD_NHWC || g->ci % 8 == 0; }
 // Its shape for P rows and Q columns: the least padded work over the shapes' relative rates (a 64-high or 64-wide tile
 // splits each staged value for half as many products).
 struct WgradSplitShape {
@@ -3361,9 +3355,9 @@ struct WgradPlan {
   int64_t slices, kslice;
 };
 // The estimate's slice count for tile ti.
-static int64_t wgrad_model_slices(const omt_conv_geo* g, int ti, int dir) {
+static int64_t wgrad_model_slices(const omt_conv_geo* g, int ti) {
   const int64_t P = g->co, Q = g->ci * g->ks * g->ks, K = g->n * g->oh * g->ow;
-  if (wgrad_is_split(dir, g, ti)) {
+  if (ti == OMT_TILE_SPLIT) {
     const WgradSplitShape& w = kWgradSplitShapes[wgrad_split_shape(P, Q)];
     const int64_t tiles = cdiv(P, w.bp) * cdiv(Q, w.bq);
     return std::max<int64_t>(1, std::min<int64_t>({kCUs / tiles, cdiv(K, 64 * 4), OMT_NOALLOC_SCRATCH_BYTES / (P * Q * 4)}));
@@ -3379,12 +3373,11 @@ static WgradPlan wgrad_plan(const omt_conv_geo* g, int dir = OMT_DIR_WGRAD) {
   int ti;
   int64_t slices;
   if (cached_plan(dir, g, &cp)) {
-    ti = cp.tile;
+    ti = cp.tile == OMT_TILE_SPLIT && !wgrad_split_ok(dir, g) ? 2 : cp.tile;
     slices = std::max<int64_t>(1, std::min<int64_t>(cp.slices, cdiv(K, 64)));
   } else {
-    const int sp = wgrad_split_tile_of(dir);
-    ti = wgrad_split_pays(P, Q, K) && wgrad_is_split(dir, g, sp) ? sp : pick_tile(kWgradTiles, P, Q, 1, kCUs * 2);
-    slices = wgrad_model_slices(g, ti, dir);
+    ti = wgrad_split_pays(P, Q, K) && wgrad_split_ok(dir, g) ? OMT_TILE_SPLIT : pick_tile(kWgradTiles, P, Q, 1, kCUs * 2);
+    slices = wgrad_model_slices(g, ti);
   }
   const int64_t kslice = cdiv(cdiv(K, slices), 64) * 64;
   return {ti, cdiv(K, kslice), kslice};
@@ -3452,12 +3445,10 @@ static bool cached_plan(int dir, const omt_conv_geo* g, omt_conv_plan* p) {
 static bool wgrad_dir(int dir) { return dir == OMT_DIR_WGRAD || dir == OMT_DIR_WGRAD_NHWC; }
 // The fp32 tiles of a direction.
 static int num_tiles(int dir) {
-  if (wgrad_dir(dir)) return dir == OMT_DIR_WGRAD_NHWC ? kWgradSplitNhwc + 1 : kWgradSplit + 1;
+  if (wgrad_dir(dir)) return kNWgrad;
   return dir == OMT_DIR_FWD_NHWC || dir == OMT_DIR_DGRAD_NHWC ? kNhwcTiles : 3 * kNGather;
 }
-static bool tile_index_ok(int dir, int t) {
-  return (t >= 0 && t < num_tiles(dir)) || (t == OMT_TILE_SPLIT && !wgrad_dir(dir));
-}
+static bool tile_index_ok(int dir, int t) { return (t >= 0 && t < num_tiles(dir)) || t == OMT_TILE_SPLIT; }
 
 }  // namespace omt
 
@@ -3938,15 +3929,15 @@ static dim3 wgrad_prepare(const omt_conv_geo* g, const float* x, const float* gy
   a.step_ox = (int)(64 % g->ow);
   a.step_oy = (int)((64 / g->ow) % g->oh);
   a.step_n = (int)((64 / g->ow) / g->oh);
-  const Tile& tl = kWgradTiles[pl.tile];
-  const bool split = wgrad_is_split(dir, g, pl.tile);
   const WgradSplitShape& sh = kWgradSplitShapes[wgrad_split_shape(a.P, a.Q)];
-  return dim3((unsigned)cdiv(a.Q, split ? sh.bq : tl.bq), (unsigned)cdiv(a.P, split ? sh.bp : tl.bp), (unsigned)pl.slices);
+  const bool split = pl.tile == OMT_TILE_SPLIT;
+  const int bp = split ? sh.bp : kWgradTiles[pl.tile].bp, bq = split ? sh.bq : kWgradTiles[pl.tile].bq;
+  return dim3((unsigned)cdiv(a.Q, bq), (unsigned)cdiv(a.P, bp), (unsigned)pl.slices);
 }
 // Tap-major column order of a grad-weight launch: each wave's BQ / 4 staged columns share one tap (split tile: its
 // units of eight columns do).
 static bool wgrad_uses_tap_major(const omt_conv_geo* g, const WgradPlan& pl) {
-  if (pl.tile == kWgradSplit) return g->ci % 8 == 0;
+  if (pl.tile == OMT_TILE_SPLIT) return g->ci % 8 == 0;
   return g->ci % (kWgradTiles[pl.tile].bq / 4) == 0;
 }
 // The grad-weight GEMM of a plan in its loader mode: 16-byte loads of four reduction pixels for 1x1 stride-1 unpadded
@@ -3954,11 +3945,11 @@ static bool wgrad_uses_tap_major(const omt_conv_geo* g, const WgradPlan& pl) {
 static void launch_wgrad_gemm(const omt_conv_geo* g, const WgradPlan& pl, const WgradArgs& a, dim3 grid,
                               hipStream_t s) {
   const bool pix4 = g->ks == 1 && g->stride == 1 && g->pad == 0 && (g->oh * g->ow) % 4 == 0;
-  if (pl.tile == kWgradSplit && pix4)
+  if (pl.tile == OMT_TILE_SPLIT && pix4)
     wgrad_split_dispatch<kPix4>(a, grid, s);
-  else if (pl.tile == kWgradSplit && wgrad_uses_tap_major(g, pl))
+  else if (pl.tile == OMT_TILE_SPLIT && wgrad_uses_tap_major(g, pl))
     wgrad_split_dispatch<kTapMajor>(a, grid, s);
-  else if (pl.tile == kWgradSplit)
+  else if (pl.tile == OMT_TILE_SPLIT)
     wgrad_split_dispatch<kGeneric>(a, grid, s);
   else if (pix4)
     wgrad_dispatch<kPix4>(pl.tile, a, grid, s);
@@ -4075,6 +4066,7 @@ OMT_EXPORT int omt_conv_wgrad_noalloc(const omt_conv_geo* g, const float* x, con
 
 // One launch for both GEMMs when their plans use the 64 x 64 tiles of conv_bwd_dual_kernel.
 static bool dual_tiles(const GatherPlan& dp, const WgradPlan& wp) {
+  if (wp.tile == OMT_TILE_SPLIT) return false;
   const Tile& gt = gtile(dp.tile);
   const Tile& wt = kWgradTiles[wp.tile];
   return gt.bp == 64 && gt.bq == 64 && gt.wp == 32 && gt.wq == 32 && (gt.bk == 16 || gt.bk == 64) && wt.bp == 64 &&
@@ -4489,7 +4481,7 @@ static int conv_wgrad_nhwc_one(const omt_conv_geo* g, const float* x, const floa
   WgradArgs a;
   WgradPlan pl;
   const dim3 grid = wgrad_prepare(g, x, gy, gw, workspace, a, pl, OMT_DIR_WGRAD_NHWC);
-  if (wgrad_is_split(OMT_DIR_WGRAD_NHWC, g, pl.tile))
+  if (pl.tile == OMT_TILE_SPLIT)
     wgrad_split_dispatch<kNhwc>(a, grid, s);
   else if (g->ci % 4 == 0)
     wgrad_nhwc_dispatch<false>(pl.tile, a, grid, s);
@@ -4621,10 +4613,13 @@ std::vector<omt_conv_plan> tune_candidates(int dir, const omt_conv_geo* g, int n
   std::vector<omt_conv_plan> out;
   if (wgrad_dir(dir)) {
     const int64_t K = g->n * g->oh * g->ow, kmax = cdiv(K, 64);
-    for (int t = 0; t < ntile; ++t) {
-      const bool split = wgrad_is_split(dir, g, t);
-      if (split && !wgrad_split_pays(g->co, g->ci * g->ks * g->ks, K)) continue;
-      const int64_t base = wgrad_model_slices(g, t, dir);
+    for (int i = 0; i <= ntile; ++i) {  // the first `ntile` tiles and, with all of them, the split tile
+      const bool split = i == ntile;
+      if (split && (ntile < num_tiles(dir) || !wgrad_split_ok(dir, g) ||
+                    !wgrad_split_pays(g->co, g->ci * g->ks * g->ks, K)))
+        break;
+      const int t = split ? OMT_TILE_SPLIT : i;
+      const int64_t base = wgrad_model_slices(g, t);
       int64_t last = -1;
       for (double m : {0.25, 0.5, 1.0, 2.0}) {
         if (split) m *= 2;  // of whole rounds of workgroups: half a round to four
@@ -4689,11 +4684,6 @@ std::vector<omt_conv_plan> tune_candidates(int dir, const omt_conv_geo* g, int n
     }
   }
   return out;
-}
-
-// Whether a plan runs a split tile.
-bool split_plan(int dir, const omt_conv_plan& p, const omt_conv_geo* g) {
-  return wgrad_dir(dir) ? wgrad_is_split(dir, g, p.tile) : gtile(p.tile).split != 0;
 }
 
 bool forcing() {
@@ -4833,7 +4823,7 @@ OMT_EXPORT int omt_conv_autotune(int dir, const omt_conv_geo* g, int max_tiles, 
   const std::vector<omt_conv_plan> cands = tune_candidates(dir, g, ntile);
   if (cands.empty()) return fail(OMT_UNSUPPORTED, "omt_conv_autotune: no candidate plan");
 
-  const bool random = std::any_of(cands.begin(), cands.end(), [&](const omt_conv_plan& c) { return split_plan(dir, c, g); });
+  const bool random = std::any_of(cands.begin(), cands.end(), [](const omt_conv_plan& c) { return c.tile == OMT_TILE_SPLIT; });
   ForceGuard guard;
   size_t ws_bytes = 0;
   for (const omt_conv_plan& c : cands) {
@@ -4900,13 +4890,14 @@ OMT_EXPORT int omt_conv_autotune_bwd(const omt_conv_geo* g, int max_tiles, void*
       if (t.bp == 64 && t.bq == 64 && t.wp == 32 && t.wq == 32 && (t.bk == 16 || t.bk == 64)) ds.push_back(d);
     }
     for (const omt_conv_plan& w : tune_candidates(OMT_DIR_WGRAD, g, wtiles)) {
+      if (w.tile == OMT_TILE_SPLIT) continue;
       const Tile& t = kWgradTiles[w.tile];
       if (t.bp == 64 && t.bq == 64 && t.wp == 32 && t.wq == 32) wsv.push_back(w);
     }
     for (const omt_conv_plan& d : ds)
       for (const omt_conv_plan& w : wsv) cands.push_back({d, w});
   }
-  const bool random = split_plan(OMT_DIR_DGRAD, dsep, g) || split_plan(OMT_DIR_WGRAD, wsep, g);
+  const bool random = dsep.tile == OMT_TILE_SPLIT || wsep.tile == OMT_TILE_SPLIT;
   ForceGuard guard;
   size_t ws_bytes = 0;
   for (const auto& c : cands) {

@@ -446,3 +446,36 @@ def test_the_split_tile_has_an_index_of_its_own():
                 assert L.omt_conv_set_plan(d, ctypes.byref(g), ctypes.byref(_lib.ConvPlan(tile, 1))) == _lib.OMT_INVALID
     finally:
         L.omt_conv_clear_plans()
+
+
+def test_split_grad_weight_index_and_untuned_plans():
+    """The four fp32 grad-weight tiles keep indices 0-3 in both memory formats, OMT_TILE_SPLIT is a plan of both
+    (channels last with input channels that are no multiple of 8 it runs as tile 2), and an untuned plan is the split
+    tile from 2^30 multiply-adds on and never below, in every direction."""
+    from omarchy_mac_torch import _lib
+    L = _lib.L
+    W, WN = _lib.OMT_DIR_WGRAD, _lib.OMT_DIR_WGRAD_NHWC
+    L.omt_conv_clear_plans()
+
+    def plan(d, g):
+        p = _lib.ConvPlan()
+        assert L.omt_conv_get_plan(d, ctypes.byref(g), ctypes.byref(p), None) == _lib.OMT_OK
+        return p.tile
+
+    try:
+        assert L.omt_conv_num_tiles(W) == L.omt_conv_num_tiles(WN) == 4
+        for ci, co in ((64, 16), (64, 32), (8, 32), (64, 512)):
+            g = _lib.conv_geo(2, ci, co, 14, 14, 3, 1, 1)
+            for d in range(6):
+                assert plan(d, g) < L.omt_conv_num_tiles(d), (d, ci, co)
+            assert plan(WN, g) == plan(W, g), (ci, co)
+        g = _lib.conv_geo(1, 512, 32, 11, 11, 11, 1, 5)
+        assert plan(WN, g) == plan(W, g) == 3  # 32 rows, 61952 columns: the fp32 32 x 128 tile
+        big = _lib.conv_geo(256, 64, 64, 56, 56, 3, 1, 1)  # 28 x 2^30
+        assert [plan(d, big) for d in range(6)] == [_lib.TILE_SPLIT] * 6
+        for ci, want in ((64, _lib.TILE_SPLIT), (60, 2)):
+            g = _lib.conv_geo(2, ci, 64, 14, 14, 3, 1, 1)
+            assert L.omt_conv_set_plan(WN, ctypes.byref(g), ctypes.byref(_lib.ConvPlan(_lib.TILE_SPLIT, 2))) == _lib.OMT_OK
+            assert plan(WN, g) == want
+    finally:
+        L.omt_conv_clear_plans()

@@ -8,7 +8,7 @@ torch = pytest.importorskip("torch")
 from oracle import oracle as orc  # noqa: E402
 
 pytestmark = pytest.mark.gpu
-SPLIT, FP32 = 256, 2  # gather tiles (OMT_TILE_SPLIT)
+SPLIT, FP32 = 256, 2  # OMT_TILE_SPLIT; the 64 x 128 gather tile
 _CL = torch.channels_last
 
 
@@ -146,7 +146,7 @@ def test_a_workgroup_redoes_all_its_tiles(cuda, ops):
     assert np.abs(a[f].astype(np.float64) - b[f]).max() <= 2 * 16 * 2.0 ** -24 * np.abs(b[f]).max()
 
 
-WSPLIT, WSPLIT_NHWC, WFP32 = 4, 3, 2  # grad-weight tiles
+WFP32 = 2  # grad-weight tile
 # rows around 64, 128 and 256, columns around 64, 128 and 256 (all five tile shapes); reductions that end inside a
 # K-block; the orders by channels: % 32 (columns by 32 channels), % 8 (tap-major), others (element by element); 1x1
 # planes of a multiple of 4 that is none of 8 (runs of four pixels that change image)
@@ -167,7 +167,7 @@ def test_split_grad_weight_is_as_exact_as_the_fp32_tile(cuda, ops, shape):
     gy = rnd(rng, *orc.conv_fwd(x, wt, None, s, p).shape)
     ref = orc.conv_wgrad(x, gy, ks, s, p)
     try:
-        for d, tile, fn in (("wgrad", WSPLIT, ops.conv2d_wgrad), ("wgrad_nhwc", WSPLIT_NHWC, ops.conv2d_wgrad_nhwc)):
+        for d, fn in (("wgrad", ops.conv2d_wgrad), ("wgrad_nhwc", ops.conv2d_wgrad_nhwc)):
             if d == "wgrad_nhwc" and co % 4:
                 continue  # not covered channels-last
             t = [torch.from_numpy(a).to(cuda) for a in (x, gy)]
@@ -175,7 +175,7 @@ def test_split_grad_weight_is_as_exact_as_the_fp32_tile(cuda, ops, shape):
             for slices in (1, 3):
                 ops.set_conv_plan(d, x.shape, wt.shape, s, p, WFP32, slices)
                 e32 = orc.rel_l2(fn(t[0], t[1], ks, s, p).contiguous().cpu().numpy(), ref)
-                ops.set_conv_plan(d, x.shape, wt.shape, s, p, tile, slices)
+                ops.set_conv_plan(d, x.shape, wt.shape, s, p, SPLIT, slices)
                 err = orc.rel_l2(fn(t[0], t[1], ks, s, p).contiguous().cpu().numpy(), ref)
                 assert err <= max(e32, 2.0 ** -24), (d, slices, err, e32)
     finally:
@@ -195,13 +195,13 @@ def test_split_grad_weight_falls_back_on_values_it_cannot_split(cuda, ops, shape
             a = x * np.float32(2.0 ** -112) if kind == "tiny" else x.copy()
             if kind == "special":
                 a[0, 3, 4, 4], a[1, 5, 2, 2] = np.inf, np.nan
-            for d, tile, fn in (("wgrad", WSPLIT, ops.conv2d_wgrad), ("wgrad_nhwc", WSPLIT_NHWC, ops.conv2d_wgrad_nhwc)):
+            for d, fn in (("wgrad", ops.conv2d_wgrad), ("wgrad_nhwc", ops.conv2d_wgrad_nhwc)):
                 if d == "wgrad_nhwc" and co % 4:
                     continue
                 t = [torch.from_numpy(v).to(cuda) for v in (a, gy)]
                 t = [v.contiguous(memory_format=_CL) for v in t] if d == "wgrad_nhwc" else t
                 got = []
-                for tl in (tile, WFP32):
+                for tl in (SPLIT, WFP32):
                     ops.set_conv_plan(d, x.shape, (co, ci, ks, ks), s, p, tl, 2)
                     got.append(fn(t[0], t[1], ks, s, p).contiguous().cpu().numpy())
                 assert np.array_equal(np.isnan(got[0]), np.isnan(got[1]))

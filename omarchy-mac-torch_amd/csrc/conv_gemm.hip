@@ -2296,7 +2296,9 @@ constexpr int wgrad_split_units() {  // of one buffer
   return MODE == kPix4 ? 12 * (BP + 4 + BQ + 4) : 3 * (BP + BQ) / 8 * kSplitBK;
 }
 
-template <int BP, int BQ, int WP, int MODE>
+// WHOLE: P is a multiple of 8, so a unit's rows are all below P or all past it; elsewhere (channels last: P % 8 == 4)
+// each row is tested, which the registers of the 128-high tiles do not have room for at no cost.
+template <int BP, int BQ, int WP, int MODE, bool WHOLE>
 __device__ __forceinline__ void wgrad_split_tile(const WgradArgs& a, const int bx, const int by, const int bz,
                                                  uint4* __restrict__ lds) {
   constexpr int NT = kSplitNT, NW = NT / 64, BK = kSplitBK, WQ = 64;
@@ -2335,18 +2337,22 @@ __device__ __forceinline__ void wgrad_split_tile(const WgradArgs& a, const int b
   // q0 + 8 (t / 32 + 16 u) .. + 7. Tap-major and channels last: the eight columns are channels of one tap. kPix4:
   // pixels 8 (t % 4) .. + 7 of gy channels p0 + t / 4 + 128 u and x channels q0 + t / 4 + 128 u.
   const int tk = t & 31, tc = t >> 5;
+  // Rows past P and columns past Q are at kOOB in the vector offset (zeros), so that no offset passes the tensors and
+  // the sums of those rows, which are not stored, stay out of split_redo. An offset below 2^31 plus kOOB is past 2^31.
   uint32_t goff[NA], xoff[NB];
-  int dy[NB], dx[NB], c0[NB];
+  int grows[NA], dy[NB], dx[NB], c0[NB];  // grows: rows of the unit below P, looked at where P % 8 != 0 (!WHOLE)
 #pragma unroll
   for (int u = 0; u < NA; ++u) {
-    const int p = p0 + 8 * (tc + 16 * u);
-    goff[u] = (uint32_t)(PIX ? (p0 + (t >> 2) + 128 * u) * ohw * 4 : MODE == kNhwc ? p * 4 : p * ohw * 4);
+    const int p = PIX ? p0 + (t >> 2) + 128 * u : p0 + 8 * (tc + 16 * u);
+    grows[u] = P - p;
+    goff[u] = p < P ? (uint32_t)(MODE == kNhwc ? p * 4 : p * ohw * 4) : kOOB;
   }
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
     const int q = q0 + 8 * (tc + 16 * u);
     if (PIX) {
-      xoff[u] = (uint32_t)((q0 + (t >> 2) + 128 * u) * HW * 4);
+      const int c = q0 + (t >> 2) + 128 * u;
+      xoff[u] = c < Q ? (uint32_t)(c * HW * 4) : kOOB;
       dy[u] = dx[u] = c0[u] = 0;
     } else if (MODE == kGeneric) {  // q = (c, ky, kx)
       const int c = (int)fdiv((uint32_t)q, a.div_kk), r = q - c * KS * KS;
@@ -2411,14 +2417,13 @@ __device__ __forceinline__ void wgrad_split_tile(const WgradArgs& a, const int b
       return;
     }
     if (v < NA) {
-      // rows past P read other rows' values, or zeros past the tensor: their sums are not stored
       const uint32_t o = gpix == kOOB ? kOOB : gpix + goff[v];
       if constexpr (MODE == kNhwc) {
-        const float4 f0 = bload4(gr, o, 0), f1 = bload4(gr, o, 16);
+        const float4 f0 = bload4(gr, o, 0), f1 = bload4(gr, WHOLE || grows[v] > 4 ? o : kOOB, 16);
         d[0] = f0.x, d[1] = f0.y, d[2] = f0.z, d[3] = f0.w, d[4] = f1.x, d[5] = f1.y, d[6] = f1.z, d[7] = f1.w;
       } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) d[e] = bload(gr, o, (uint32_t)(e * ohw * 4));
+        for (int e = 0; e < 8; ++e) d[e] = bload(gr, WHOLE || e < grows[v] ? o : kOOB, (uint32_t)(e * ohw * 4));
       }
       return;
     }
@@ -2599,11 +2604,11 @@ __device__ __forceinline__ void wgrad_split_tile(const WgradArgs& a, const int b
   }
 }
 
-template <int BP, int BQ, int WP, int MODE>
+template <int BP, int BQ, int WP, int MODE, bool WHOLE>
 __global__ void __launch_bounds__(kSplitNT, 2) conv_wgrad_split_kernel(const WgradArgs a) {
   __shared__ __attribute__((aligned(16))) uint4 lds[2 * wgrad_split_units<BP, BQ, MODE>()];
   const TileId t = xcd_block_tile(kTileGroup);
-  wgrad_split_tile<BP, BQ, WP, MODE>(a, t.x, t.y, t.z, lds);
+  wgrad_split_tile<BP, BQ, WP, MODE, WHOLE>(a, t.x, t.y, t.z, lds);
 }
 
 // Grad input and grad weight of one convolution in one launch (omt_conv_bwd), both on 64 x 64 tiles: the first
@@ -3393,15 +3398,22 @@ static void wgrad_dispatch(int ti, const WgradArgs& a, dim3 grid, hipStream_t s)
   }
 }
 
+template <int MODE, bool WHOLE>
+static void wgrad_split_launch(const WgradArgs& a, dim3 grid, hipStream_t s) {
+  switch (wgrad_split_shape(a.P, a.Q)) {
+    case 0: hipLaunchKernelGGL((conv_wgrad_split_kernel<128, 256, 64, MODE, WHOLE>), grid, dim3(kSplitNT), 0, s, a); break;
+    case 1: hipLaunchKernelGGL((conv_wgrad_split_kernel<256, 128, 64, MODE, WHOLE>), grid, dim3(kSplitNT), 0, s, a); break;
+    case 2: hipLaunchKernelGGL((conv_wgrad_split_kernel<128, 128, 32, MODE, WHOLE>), grid, dim3(kSplitNT), 0, s, a); break;
+    case 3: hipLaunchKernelGGL((conv_wgrad_split_kernel<64, 256, 32, MODE, WHOLE>), grid, dim3(kSplitNT), 0, s, a); break;
+    default: hipLaunchKernelGGL((conv_wgrad_split_kernel<256, 64, 32, MODE, WHOLE>), grid, dim3(kSplitNT), 0, s, a); break;
+  }
+}
 template <int MODE>
 static void wgrad_split_dispatch(const WgradArgs& a, dim3 grid, hipStream_t s) {
-  switch (wgrad_split_shape(a.P, a.Q)) {
-    case 0: hipLaunchKernelGGL((conv_wgrad_split_kernel<128, 256, 64, MODE>), grid, dim3(kSplitNT), 0, s, a); break;
-    case 1: hipLaunchKernelGGL((conv_wgrad_split_kernel<256, 128, 64, MODE>), grid, dim3(kSplitNT), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((conv_wgrad_split_kernel<128, 128, 32, MODE>), grid, dim3(kSplitNT), 0, s, a); break;
-    case 3: hipLaunchKernelGGL((conv_wgrad_split_kernel<64, 256, 32, MODE>), grid, dim3(kSplitNT), 0, s, a); break;
-    default: hipLaunchKernelGGL((conv_wgrad_split_kernel<256, 64, 32, MODE>), grid, dim3(kSplitNT), 0, s, a); break;
-  }
+  if (MODE == kPix4 || a.P % 8 == 0)  // kPix4's threads load one row each
+    wgrad_split_launch<MODE, true>(a, grid, s);
+  else if constexpr (MODE != kPix4)
+    wgrad_split_launch<MODE, false>(a, grid, s);
 }
 
 template <bool NARROW>

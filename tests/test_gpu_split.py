@@ -157,6 +157,45 @@ WSHAPES = [
 ]
 
 
+# a last unit of gy rows that is not whole: P % 8 != 0 (channels last P % 8 == 4), few rows and one past a tile's edge,
+# one image, in each column order
+ROW_EDGES = [
+    (1, 32, 1, 12, 11, 3, 1, 1), (1, 24, 3, 12, 11, 3, 1, 1), (1, 12, 5, 9, 13, 3, 2, 1), (1, 64, 3, 8, 9, 1, 1, 0),
+    (1, 40, 4, 9, 9, 3, 1, 1), (1, 32, 12, 12, 11, 3, 1, 1), (1, 32, 129, 7, 7, 3, 1, 1), (1, 32, 132, 7, 7, 3, 1, 1),
+    (1, 300, 68, 7, 7, 1, 1, 0),
+]
+
+
+@pytest.mark.parametrize("shape", ROW_EDGES, ids=lambda s: "x".join(map(str, s)))
+def test_split_grad_weight_reads_no_row_past_the_last(cuda, ops, shape):
+    """gy lies in front of NaNs in one allocation: a row past gy's last, though not stored, would have the tile computed
+    again in fp32, whose sums differ. The result is that of gy alone, to the bit, and as exact as the fp32 tile's."""
+    n, ci, co, h, w, ks, s, p = shape
+    rng = np.random.default_rng(sum(shape) + 3)
+    x, wt = rnd(rng, n, ci, h, w), rnd(rng, co, ci, ks, ks)
+    gy = rnd(rng, *orc.conv_fwd(x, wt, None, s, p).shape)
+    ref = orc.conv_wgrad(x, gy, ks, s, p)
+    try:
+        for d, fn in (("wgrad", ops.conv2d_wgrad), ("wgrad_nhwc", ops.conv2d_wgrad_nhwc)):
+            nhwc = d == "wgrad_nhwc"
+            if nhwc and (co % 4 or ci % 8):
+                continue
+            tx, tg = (torch.from_numpy(a).to(cuda).contiguous(memory_format=_CL if nhwc else torch.contiguous_format)
+                      for a in (x, gy))
+            buf = torch.full((gy.size + 8 * gy[0, 0].size + 64,), float("nan"), device=cuda)
+            view = buf[:gy.size].view(n, *gy.shape[2:], co).permute(0, 3, 1, 2) if nhwc else buf[:gy.size].view(gy.shape)
+            view.copy_(tg)
+            got = []
+            for tile, g in ((SPLIT, tg), (SPLIT, view), (WFP32, tg)):
+                ops.set_conv_plan(d, x.shape, wt.shape, s, p, tile, 1)
+                got.append(fn(tx, g, ks, s, p).contiguous().cpu().numpy())
+            assert np.array_equal(got[0], got[1]), d
+            err, e32 = orc.rel_l2(got[0], ref), orc.rel_l2(got[2], ref)
+            assert err <= max(e32, 2.0 ** -24), (d, err, e32)
+    finally:
+        ops.clear_conv_plans()
+
+
 @pytest.mark.parametrize("shape", WSHAPES, ids=lambda s: "x".join(map(str, s)))
 def test_split_grad_weight_is_as_exact_as_the_fp32_tile(cuda, ops, shape):
     """Both memory formats, 1 and 3 K slices, against the float64 oracle: off by no more than the fp32 tile, or one

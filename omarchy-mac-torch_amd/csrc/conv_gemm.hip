@@ -812,7 +812,10 @@ __device__ __forceinline__ bool split_redo(const omt_f32x4 (&acc)[TI][TJ], int w
 #pragma unroll
     for (int j = 0; j < TJ; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) m = max(m, __builtin_bit_cast(uint32_t, acc[i][j][r]) & 0x7fffffffu);
+      for (int r = 0; r < 4; ++r) {
+        const float v = acc[i][j][r];  // (a bit cast of a vector's element itself is compiled as its first element)
+        m = max(m, __builtin_bit_cast(uint32_t, v) & 0x7fffffffu);
+      }
   constexpr uint32_t kTiny = (127u - 60u) << 23;  // 2^-60
   const uint32_t bits = (__ballot(m >= 0x7f800000u) ? 1u : 0u) | (__ballot(m >= kTiny) ? 2u : 0u) |
                         (__ballot(m != 0) ? 4u : 0u);

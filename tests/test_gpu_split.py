@@ -130,6 +130,38 @@ def test_split_tile_falls_back_on_values_it_cannot_split(cuda, ops, kind, ci):
         ops.clear_conv_plans()
 
 
+@pytest.mark.parametrize("val", [np.inf, np.nan, 3.4e38], ids=str)
+def test_one_sum_anywhere_in_a_tile_calls_for_fp32(cuda, ops, val):
+    """A value that the split cannot carry in one row of the filter (or of gy), each place of a lane's four accumulator
+    rows in turn: the outputs are the fp32 tile's, NaN, infinity or finite, and to the bit (one 16-deep order)."""
+    rng = np.random.default_rng(5)
+    n, ci, co, h = 1, 64, 64, 8
+    x, wt, gy = rnd(rng, n, ci, h, h), rnd(rng, co, ci, 3, 3, scale=0.05), rnd(rng, n, co, h, h)
+    try:
+        for row in (0, 17, 34, 63):
+            for d in ("fwd", "dgrad", "fwd_nhwc", "dgrad_nhwc", "wgrad", "wgrad_nhwc"):
+                xv, wv, gv = x.copy(), wt.copy(), gy.copy()
+                if d.startswith("wgrad"):
+                    gv[0, row, 3, 4] = val
+                elif d.startswith("dgrad"):
+                    wv[5, row, 1, 1] = val
+                else:
+                    wv[row, 5, 1, 1] = val
+                t = [torch.from_numpy(a).to(cuda) for a in (xv, wv, gv)]
+                t = [a.contiguous(memory_format=_CL) for a in t] if d.endswith("nhwc") else t
+                got = []
+                for tile in (SPLIT, FP32):
+                    if d.startswith("wgrad"):
+                        ops.set_conv_plan(d, x.shape, wt.shape, 1, 1, tile, 1)
+                        fn = ops.conv2d_wgrad_nhwc if d.endswith("nhwc") else ops.conv2d_wgrad
+                        got.append(fn(t[0], t[2], 3, 1, 1).contiguous().cpu().numpy())
+                    else:
+                        got.append(run(ops, d, t, xv, wv, gv, 1, 1, tile))
+                assert np.array_equal(*got, equal_nan=True), (row, d)
+    finally:
+        ops.clear_conv_plans()
+
+
 def test_a_workgroup_redoes_all_its_tiles(cuda, ops):
     """283 tiles on 256 CUs: a NaN in one of them has its workgroup compute all its tiles again in fp32."""
     rng = np.random.default_rng(11)

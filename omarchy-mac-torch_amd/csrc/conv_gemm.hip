@@ -995,7 +995,8 @@ __device__ __forceinline__ void gather_split_tiles(const GatherArgs& a, const in
   SplitTiles at = cur;
   int ak = 0;
   auto aload = [&](const int buf) {
-    const uint32_t src = (uint32_t)((ph.soff + (at.t.y * ph.snkb + kbeg / BK + ak) * 12 * BP) * 16);
+    // an empty slice's K-block lies past the phase's: it takes the last one, against zeros of x
+    const uint32_t src = (uint32_t)((ph.soff + (at.t.y * ph.snkb + min(kbeg / BK + ak, ph.snkb - 1)) * 12 * BP) * 16);
 #pragma unroll
     for (int i = 0; i < (AKB + NW - 1) / NW; ++i) {
       const int c = wave + NW * i;

@@ -68,6 +68,33 @@ def test_split_tile_is_as_exact_as_the_fp32_tile(cuda, ops, shape):
         ops.clear_conv_plans()
 
 
+@pytest.mark.parametrize("shape", [(1, 130, 128, 5, 5, 3, 2, 1), (2, 64, 96, 7, 4, 5, 3, 2), (1, 96, 40, 3, 9, 3, 4, 1), (1, 64, 128, 7, 7, 3, 2, 0)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_split_k_slices_past_a_short_phase(cuda, ops, shape):
+    """A strided grad input's phases sum one tap to several (or none): in as many K slices as the longest has K-blocks,
+    most slices of the short ones are empty. Against the oracle; and with an infinity and a NaN in the filter, which
+    reach the pixels that they reach through the fp32 tile."""
+    n, ci, co, h, w, ks, s, p = shape
+    rng = np.random.default_rng(sum(shape))
+    x, wt = rnd(rng, n, ci, h, w), rnd(rng, co, ci, ks, ks)
+    gy = rnd(rng, n, co, (h + 2 * p - ks) // s + 1, (w + 2 * p - ks) // s + 1)
+    ref = orc.conv_dgrad(gy, wt, x.shape, s, p)
+    try:
+        for special in (False, True):
+            if special:
+                wt[co - 1, ci - 1, 1, 1], wt[3, 5, 0, 2] = np.inf, np.nan
+            t = [torch.from_numpy(a).to(cuda) for a in (x, wt, gy)]
+            tc = [a.contiguous(memory_format=_CL) for a in t]
+            for d, u in (("dgrad", t), ("dgrad_nhwc", tc)):
+                for slices in (3, 64):
+                    a, b = (run(ops, d, u, x, wt, gy, s, p, tile, slices) for tile in (SPLIT, FP32))
+                    assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b))
+                    if not special:
+                        assert orc.rel_l2(a, ref) <= max(orc.rel_l2(b, ref), 2.0 ** -24), (d, slices)
+    finally:
+        ops.clear_conv_plans()
+
+
 @pytest.mark.parametrize("shape", [(2, 32, 130, 9, 15, 3, 1, 1), (3, 48, 64, 10, 7, 3, 2, 1), (2, 64, 140, 8, 8, 1, 1, 0)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_tile_1_is_the_fp32_128x128_tile(cuda, ops, shape):

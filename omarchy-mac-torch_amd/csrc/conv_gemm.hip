@@ -700,24 +700,32 @@ __device__ __forceinline__ void gather_tile(const GatherArgs& a, const int bx, c
 }
 
 // ---- split-bf16 gather tiles --------------------------------------------------------------------------------------
-// Tile 1 runs fp32 products on the bf16 matrix cores. Each float is split into three bf16 terms x = h + m + l (round
-// to nearest each time: 24 significant bits, so the split is exact but for terms below the smallest bf16 subnormal),
-// and a product keeps the six partial products above 2^-24 of it: hh, hm + mh, mm, hl + lh (those left out are at
-// most 2^-26 of hh each). bf16 products are exact in the matrix core's fp32 accumulator. Six
-// v_mfma_f32_16x16x32_bf16 (1950 TFLOP/s dense here on random data) do the work of eight v_mfma_f32_16x16x4_f32
-// (146 TFLOP/s): 2.2 times the rate.
+// The split tile (OMT_TILE_SPLIT) runs fp32 products on the bf16 matrix cores. Each float is split into three bf16 terms
+// x = h + m + l (round to nearest each time: 24 significant bits, so the split is exact but for the smallest floats, see
+// below), and a product keeps the six largest of the nine partial products: hh, hm + mh, mm, hl + lh. Of the three left
+// out, ml and lm are at most 2^-25 of the product each and ll 2^-34: 2^-24 together at worst (both operands
+// 1 + 2^-8 - 2^-17), half a unit in the last place of the product. bf16 products are exact in the matrix core's fp32
+// accumulator. Six v_mfma_f32_16x16x32_bf16 (1950 TFLOP/s dense here on random data) do the work of eight
+// v_mfma_f32_16x16x4_f32 (146 TFLOP/s): 2.2 times the rate.
 // Accuracy: each 32-deep K-block is summed from zero, smallest partial products first, and added to the running sum
 // with one fp32 add, so the running sum is rounded once per 32 products, where the fp32 instruction rounds it per
 // product. Against float64 sums of random products the relative error is 0.9e-7 at K 576 and 2.4e-7 at K 4608; the
 // fp32 MFMA chain has 3.0-4.4e-7 and 0.9-1.2e-6.
 // Range: a value whose split overflows (infinite, NaN, or within 2^-9 of the largest float), or an overflowing sum,
-// leaves a non-finite accumulator; inputs so small that their low terms underflow leave only tiny ones. A tile that
-// holds a non-finite sum, or whose largest sum is below 2^-60 and not zero, is computed again by the fp32 tile
-// (split_redo), so such inputs give what the fp32 instructions give.
+// leaves a non-finite accumulator. A value whose last term is below 2^-126 (it may round in bf16 there) is seen where
+// it is split: in the source by a test of that term, whatever else the tile holds and however large the other operand;
+// in the filter by the pack, which then makes h NaN. A workgroup that meets one of these, or whose largest sum is below
+// 2^-60 and not zero, computes its tiles again by the fp32 tile (split_redo), so such inputs give what the fp32
+// instructions give.
 typedef __bf16 omt_bf16x8 __attribute__((ext_vector_type(8)));
 
-// Terms h, m, l of two floats, each pair packed as two bf16 (x in the low half).
-__device__ __forceinline__ void split_bf16(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
+// Terms h, m, l of two floats, each pair packed as two bf16 (x in the low half). The rest after h and m has at most 8
+// significant bits, so l is exact unless the rest is subnormal: `least` becomes the least over the rests seen of twice
+// the magnitude's bits, less one (a rest of zero is the largest), and is below kLost where one was subnormal. (As fp
+// class tests, one VALU instruction and one scalar one a value, the grad weight took 4-13% more time; so, 1.5 VALU
+// instructions, it takes 3-4% and the gather tiles 0.5-2% more than without the test.)
+constexpr uint32_t kLost = 0xffffffu;
+__device__ __forceinline__ void split_bf16(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l, uint32_t& least) {
   // (through the conversion in C++ the compiler converts some terms twice, once packed and once alone)
   const auto pack = [](float a, float b) {
     uint32_t r;
@@ -729,7 +737,10 @@ __device__ __forceinline__ void split_bf16(float x, float y, uint32_t& h, uint32
   h = pack(x, y);
   const float x1 = x - lo(h), y1 = y - hi(h);
   m = pack(x1, y1);
-  l = pack(x1 - lo(m), y1 - hi(m));
+  float x2 = x1 - lo(m), y2 = y1 - hi(m);  // (by hand so that the rests' registers are used up here)
+  asm("v_cvt_pk_bf16_f32 %0, %2, %3\n\tv_lshl_add_u32 %2, %2, 1, -1\n\tv_lshl_add_u32 %3, %3, 1, -1\n\t"
+      "v_min3_u32 %1, %1, %2, %3"
+      : "=&v"(l), "+v"(least), "+v"(x2), "+v"(y2));
 }
 
 // A K-block of 32 k of R rows is staged as 16-byte units of 8 k of one row and one term, unit (term z, k group g,
@@ -740,7 +751,8 @@ constexpr int kSplitNT = 512;                 // threads of a workgroup (one per
 constexpr int kSplitBQ = 256;                 // columns of a gather tile
 
 // The filter, packed for the split tile: for each phase, tile of BP rows and K-block, the K-block's units in LDS
-// order, rows past P and k past K zero. One thread per (row, 8 k): three units.
+// order, rows past P and k past K zero. One thread per (row, 8 k): three units; where one of the eight does not split
+// exactly, NaN among them.
 template <int BP>
 __global__ void __launch_bounds__(256) split_pack_kernel(const GatherArgs a, uint4* __restrict__ out, int nunits) {
   const int u = blockIdx.x * 256 + threadIdx.x;
@@ -772,8 +784,10 @@ __global__ void __launch_bounds__(256) split_pack_kernel(const GatherArgs a, uin
     v[e] = p < a.P && k < ph.K ? a.w[off / 4] : 0.f;
   }
   uint32_t h[4], m[4], l[4];
+  uint32_t least = ~0u;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) split_bf16(v[2 * e], v[2 * e + 1], h[e], m[e], l[e]);
+  for (int e = 0; e < 4; ++e) split_bf16(v[2 * e], v[2 * e + 1], h[e], m[e], l[e], least);
+  if (least < kLost) h[0] = 0x7fc07fc0u;  // NaN: this row's tiles are computed again in fp32
   uint4* const o = out + ph.soff + (int64_t)blk * 12 * BP + g * BP + row;
   o[0] = make_uint4(h[0], h[1], h[2], h[3]);
   o[4 * BP] = make_uint4(m[0], m[1], m[2], m[3]);
@@ -802,11 +816,15 @@ struct SplitTiles {
   __device__ __forceinline__ TileId at(int ntiles) const { return xcd_tile(pid, gx, gy, ntiles / (gx * gy), kTileGroup); }
 };
 
-// Whether a workgroup's finished sums call for the fp32 tile (see above), the same answer in every thread. Uses a
-// dword of LDS per wave at `flags` that no wave still reads; returns after a barrier, with `flags` free again.
+// Whether a workgroup's finished sums, or the lanes `lost` whose source values did not split exactly, call for the fp32
+// tile (see above), the same answer in every thread. Uses a dword of LDS per wave at `flags` that no wave still reads;
+// returns after a barrier, with `flags` free again.
 template <int TI, int TJ, int NW>
-__device__ __forceinline__ bool split_redo(const omt_f32x4 (&acc)[TI][TJ], int wave, int lane, uint32_t* flags) {
-  uint32_t m = 0;
+__device__ __forceinline__ bool split_redo(const omt_f32x4 (&acc)[TI][TJ], uint64_t lost, int wave, int lane,
+                                           uint32_t* flags) {
+  // the largest sum's bits: of the positive ones the largest as a signed integer, of the negative as an unsigned one
+  int pos = 0;
+  uint32_t neg = 0;
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -814,10 +832,12 @@ __device__ __forceinline__ bool split_redo(const omt_f32x4 (&acc)[TI][TJ], int w
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float v = acc[i][j][r];  // (a bit cast of a vector's element itself is compiled as its first element)
-        m = max(m, __builtin_bit_cast(uint32_t, v) & 0x7fffffffu);
+        pos = max(pos, __builtin_bit_cast(int, v));
+        neg = max(neg, __builtin_bit_cast(uint32_t, v));
       }
+  const uint32_t m = max((uint32_t)pos, neg >> 31 ? neg & 0x7fffffffu : 0u);
   constexpr uint32_t kTiny = (127u - 60u) << 23;  // 2^-60
-  const uint32_t bits = (__ballot(m >= 0x7f800000u) ? 1u : 0u) | (__ballot(m >= kTiny) ? 2u : 0u) |
+  const uint32_t bits = (__ballot(m >= 0x7f800000u) | lost ? 1u : 0u) | (__ballot(m >= kTiny) ? 2u : 0u) |
                         (__ballot(m != 0) ? 4u : 0u);
   if (lane == 0) flags[wave] = bits;
   __syncthreads();
@@ -1013,10 +1033,11 @@ __device__ __forceinline__ void gather_split_tiles(const GatherArgs& a, const in
 
   // A quarter of this thread's source values: split four k, and store each eight as three units.
   uint32_t sh[4], sm[4], sl[4];
+  uint32_t least = ~0u;
   auto sstore = [&](const int quarter, const int buf) {
     const int e = 4 * quarter, u = 2 * (quarter & 1);
-    split_bf16(rb[e], rb[e + 1], sh[u], sm[u], sl[u]);
-    split_bf16(rb[e + 2], rb[e + 3], sh[u + 1], sm[u + 1], sl[u + 1]);
+    split_bf16(rb[e], rb[e + 1], sh[u], sm[u], sl[u], least);
+    split_bf16(rb[e + 2], rb[e + 3], sh[u + 1], sm[u + 1], sl[u + 1], least);
     if (quarter & 1) {
       const int g = MODE == kNhwc ? cg : rbase / 8 + quarter / 2;
       const int row = MODE == kNhwc ? t / 4 + 128 * (quarter / 2) : t % BQ;
@@ -1104,7 +1125,7 @@ __device__ __forceinline__ void gather_split_tiles(const GatherArgs& a, const in
     }
     // the next tile's first K-block waits in buffer `buf`; the other one is free for the epilogue
     float* const fl = reinterpret_cast<float*>(lds + (buf ^ 1) * BUF);
-    redo |= split_redo<TI, TJ, NW>(acc, wave, lane, reinterpret_cast<uint32_t*>(fl));
+    redo |= split_redo<TI, TJ, NW>(acc, __ballot(least < kLost), wave, lane, reinterpret_cast<uint32_t*>(fl));
     split_epilogue<BP, BQ, WP, WQ, MODE>(a, ph, acc, cur.t.x, cur.t.y, zs, wave, lane, fl);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(63) & ~0xF00);
@@ -1207,12 +1228,13 @@ __device__ __forceinline__ void gather_window_tile(const GatherArgs& a, const in
       }
     }
   };
+  uint32_t least = ~0u;
   auto sstore = [&]() {
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
       uint32_t h[4], m[4], l[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) split_bf16(rb[u][2 * e], rb[u][2 * e + 1], h[e], m[e], l[e]);
+      for (int e = 0; e < 4; ++e) split_bf16(rb[u][2 * e], rb[u][2 * e + 1], h[e], m[e], l[e], least);
       if (s0 + NT / 4 * u < slots) {
         uint4* const o = Bs + g * NS + s0 + NT / 4 * u;
         o[0] = make_uint4(h[0], h[1], h[2], h[3]);
@@ -1339,7 +1361,7 @@ __device__ __forceinline__ void gather_window_tile(const GatherArgs& a, const in
 
   static_assert(NW * row_epi_floats<WQ>() <= 4 * 12 * NS && gather_lds_floats<64, 128, 16>() <= 4 * 12 * NS, "LDS");
   float* const fl = reinterpret_cast<float*>(lds);
-  if (split_redo<TI, TJ, NW>(acc, wave, lane, reinterpret_cast<uint32_t*>(lds)))
+  if (split_redo<TI, TJ, NW>(acc, __ballot(least < kLost), wave, lane, reinterpret_cast<uint32_t*>(lds)))
     split_redo_tiles<BP, BQ, MODE>(a, ntiles, wave, fl);
   else
     split_epilogue<BP, BQ, WP, WQ, MODE>(a, ph, acc, tile.x, tile.y, 0, wave, lane, fl);
@@ -2458,10 +2480,11 @@ __device__ __forceinline__ void wgrad_split_tile(const WgradArgs& a, const int b
       }
     }
   };
+  uint32_t least = ~0u;
   auto sstore = [&](const int v, const int buf) {
     uint32_t h[4], m[4], l[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) split_bf16(rv[v][2 * e], rv[v][2 * e + 1], h[e], m[e], l[e]);
+    for (int e = 0; e < 4; ++e) split_bf16(rv[v][2 * e], rv[v][2 * e + 1], h[e], m[e], l[e], least);
     const int u = v < NA ? v : v - NA, c = tc + 16 * u;
     const int term = PIX ? 4 * ((v < NA ? BP : BQ) + 4) : (v < NA ? AC : BC) * BK;  // units from one term to the next
     uint4* const o = lds + buf * BUF + (v < NA ? 0 : 3 * (PIX ? 4 * (BP + 4) : AC * BK)) +
@@ -2563,7 +2586,7 @@ __device__ __forceinline__ void wgrad_split_tile(const WgradArgs& a, const int b
   if (it < nk) step(it, std::integral_constant<int, 0>{});
 
   float* const fl = reinterpret_cast<float*>(lds);
-  if (split_redo<TI, TJ, NW>(acc, wave, lane, reinterpret_cast<uint32_t*>(lds))) {
+  if (split_redo<TI, TJ, NW>(acc, __ballot(least < kLost), wave, lane, reinterpret_cast<uint32_t*>(lds))) {
     // the fp32 tile is the work of four waves; a barrier waits for the waves that have not ended
     if (wave >= 4) return;
     constexpr int FP = BP / 64, FQ = BQ / 32;

@@ -189,6 +189,136 @@ def test_one_sum_anywhere_in_a_tile_calls_for_fp32(cuda, ops, val):
         ops.clear_conv_plans()
 
 
+def run_dir(ops, d, a, s, p, tile, slices=1):
+    """Direction d of the layer with host arrays a = (x, w, gy) under the plan (tile, slices)."""
+    t = [torch.from_numpy(np.ascontiguousarray(v)).to("cuda") for v in a]
+    t = [v.contiguous(memory_format=_CL) for v in t] if d.endswith("nhwc") else t
+    if not d.startswith("wgrad"):
+        return run(ops, d, t, *a, s, p, tile, slices)
+    ops.set_conv_plan(d, a[0].shape, a[1].shape, s, p, tile, slices)
+    fn = ops.conv2d_wgrad_nhwc if d.endswith("nhwc") else ops.conv2d_wgrad
+    return fn(t[0], t[2], a[1].shape[2], s, p).contiguous().cpu().numpy()
+
+
+ALL_DIRS = ("fwd", "dgrad", "wgrad", "fwd_nhwc", "dgrad_nhwc", "wgrad_nhwc")
+# one tile each: window, split, channel-major, strided phases, super-pixel grad input, 1x1
+ONE_TILE = [(2, 64, 64, 8, 8, 3, 1, 1), (2, 48, 64, 8, 8, 3, 1, 1), (2, 33, 40, 8, 8, 3, 1, 1), (2, 48, 64, 9, 9, 3, 2, 1),
+            (2, 3, 32, 33, 29, 11, 4, 2), (2, 64, 64, 8, 8, 1, 1, 0)]
+
+
+@pytest.mark.parametrize("kind", ["huge_x", "huge_w", "tiny_image", "tiny_row", "subnormal"])
+@pytest.mark.parametrize("shape", ONE_TILE, ids=lambda s: "x".join(map(str, s)))
+def test_operands_that_lose_bits_in_the_split(cuda, ops, shape, kind):
+    """Operands below 2^-109 lose bits in bf16, which shows in no sum where the other operand is huge or the rest of the
+    tile is ordinary. Every direction gives the fp32 tile's outputs, to the bit (the whole tile is computed again)."""
+    n, ci, co, h, w, ks, s, p = shape
+    rng = np.random.default_rng(sum(shape))
+    x, wt = rnd(rng, n, ci, h, w), rnd(rng, co, ci, ks, ks)
+    gy = rnd(rng, n, co, (h + 2 * p - ks) // s + 1, (w + 2 * p - ks) // s + 1)
+    up, down = np.float32(2.0 ** 100), np.float32(2.0 ** -119)
+    try:
+        for d in ALL_DIRS:
+            if d == "wgrad_nhwc" and (co % 4 or ci % 8) or d == "fwd_nhwc" and ci % 16 or d == "dgrad_nhwc" and co % 16:
+                continue  # not the split tile
+            a = [x.copy(), wt.copy(), gy.copy()]
+            # the operands: source and filter, or the two sources of the grad weight
+            i, j = {"f": (0, 1), "d": (2, 1), "w": (0, 2)}[d[0]]
+            if kind in ("huge_x", "huge_w"):
+                i, j = (i, j) if kind == "huge_x" else (j, i)
+                a[i] *= up
+                a[j] *= down
+            elif kind == "tiny_image":
+                a[i][0] *= down
+            elif kind == "tiny_row":  # of the filter's output rows; of gy
+                if j == 1 and d[0] == "f":
+                    a[1][5] *= down
+                else:
+                    a[j][:, 2] *= down
+            else:
+                a[i] *= np.float32(2.0 ** -110)
+                a[i] *= np.float32(2.0 ** -28)
+                a[j] *= np.float32(2.0 ** 110)
+            slices = 2 if d[0] == "w" and kind != "tiny_image" else 1  # (an ordinary image's slice stays split)
+            got = [run_dir(ops, d, a, s, p, tile, slices) for tile in (SPLIT, FP32)]
+            assert np.array_equal(*got), d
+            if kind != "subnormal" or d[0] == "w":
+                assert np.abs(got[1]).max() > 0, d
+    finally:
+        ops.clear_conv_plans()
+
+
+@pytest.mark.parametrize("shape", ONE_TILE, ids=lambda s: "x".join(map(str, s)))
+def test_small_operands_that_split_exactly(cuda, ops, shape):
+    """Multiples k 2^-130, |k| <= 5, are subnormal in bf16 and split exactly: against integers times 2^90 every sum is
+    exact in fp32, and so is the split tile's (no test calls for the fp32 tile)."""
+    n, ci, co, h, w, ks, s, p = shape
+    rng = np.random.default_rng(sum(shape))
+    oh, ow = (h + 2 * p - ks) // s + 1, (w + 2 * p - ks) // s + 1
+    ints = [rng.integers(-5, 6, sh).astype(np.float64) for sh in ((n, ci, h, w), (co, ci, ks, ks), (n, co, oh, ow))]
+    ref = [orc.conv_fwd(*(v.astype(np.float32) for v in ints[:2]), None, s, p),
+           orc.conv_dgrad(ints[2].astype(np.float32), ints[1].astype(np.float32), ints[0].shape, s, p),
+           orc.conv_wgrad(ints[0].astype(np.float32), ints[2].astype(np.float32), ks, s, p)]
+    try:
+        for d in ALL_DIRS:
+            if d == "wgrad_nhwc" and (co % 4 or ci % 8) or d == "fwd_nhwc" and ci % 16 or d == "dgrad_nhwc" and co % 16:
+                continue
+            i, j, r = {"f": (0, 1, 0), "d": (2, 1, 1), "w": (0, 2, 2)}[d[0]]
+            for lo, hi in ((i, j), (j, i)):
+                a = [v.astype(np.float32) for v in ints]
+                a[lo] = (ints[lo] * 2.0 ** -130).astype(np.float32)
+                a[hi] = (ints[hi] * 2.0 ** 90).astype(np.float32)
+                got = run_dir(ops, d, a, s, p, SPLIT)
+                assert np.array_equal(got * np.float32(2.0 ** 40), np.asarray(ref[r], np.float32)), (d, lo)
+    finally:
+        ops.clear_conv_plans()
+
+
+@pytest.mark.parametrize("shape", ONE_TILE[:4], ids=lambda s: "x".join(map(str, s)))
+def test_products_that_underflow_beside_ordinary_ones(cuda, ops, shape):
+    """One image and one filter row at 2^-70: their products are subnormal in a tile whose other sums are ordinary. Each
+    output is within K 2^-24 of its sum of magnitudes, and K of the smallest float, of the exact one."""
+    n, ci, co, h, w, ks, s, p = shape
+    rng = np.random.default_rng(sum(shape))
+    x, wt = rnd(rng, n, ci, h, w), rnd(rng, co, ci, ks, ks)
+    x[0] *= np.float32(2.0 ** -70)
+    wt[3] *= np.float32(2.0 ** -70)
+    gy = np.zeros((n, co, (h + 2 * p - ks) // s + 1, (w + 2 * p - ks) // s + 1), np.float32)
+    tx, tw = torch.from_numpy(x).double(), torch.from_numpy(wt).double()
+    ref = torch.nn.functional.conv2d(tx, tw, None, s, p).numpy()
+    mag = torch.nn.functional.conv2d(tx.abs(), tw.abs(), None, s, p).numpy()
+    k = ci * ks * ks
+    try:
+        for d in ("fwd", "fwd_nhwc"):
+            if d == "fwd_nhwc" and ci % 16:
+                continue
+            got = run_dir(ops, d, [x, wt, gy], s, p, SPLIT).astype(np.float64)
+            assert (np.abs(got - ref) <= k * (2.0 ** -24 * mag + 2.0 ** -149)).all(), d
+    finally:
+        ops.clear_conv_plans()
+
+
+def test_the_worst_operands_of_the_kept_products(cuda, ops):
+    """1 + 2^-8 - 2^-17 = h + m + l with the largest m and l: the partial products left out are 2^-24 of each product,
+    with one sign. Beside them at most one rounding (2^-24, relative) for each matrix instruction of a K-block (6) and
+    for each K-block's addition."""
+    v = np.float32(1 + 2.0 ** -8 - 2.0 ** -17)
+    try:
+        for n, ci, co, h, ks, p in ((1, 64, 64, 16, 3, 1), (1, 48, 64, 16, 1, 0), (1, 128, 130, 16, 1, 0)):
+            a = [np.full((n, ci, h, h), v), np.full((co, ci, ks, ks), v), np.full((n, co, h, h), v)]
+            taps = np.ones((1, 1, ks, ks), np.float32)
+            count = orc.conv_fwd(np.ones((n, 1, h, h), np.float32), taps, None, 1, p).astype(np.float64)  # taps inside
+            for d, ref, k in (("fwd", count * ci, ci * ks * ks), ("dgrad", count * co, co * ks * ks),
+                              ("wgrad", None, h * h)):
+                got = run_dir(ops, d, a, 1, p, SPLIT).astype(np.float64)
+                if d == "wgrad":
+                    side = np.array([h - abs(i - ks // 2) for i in range(ks)], np.float64)
+                    ref = np.outer(side, side)
+                exact = ref * float(v) ** 2
+                assert (np.abs(got - exact) <= (1 + 6 + -(-k // 32)) * 2.0 ** -24 * exact).all(), d
+    finally:
+        ops.clear_conv_plans()
+
+
 def test_a_workgroup_redoes_all_its_tiles(cuda, ops):
     """283 tiles on 256 CUs: a NaN in one of them has its workgroup compute all its tiles again in fp32."""
     rng = np.random.default_rng(11)

@@ -3221,9 +3221,7 @@ static bool wst_ok(const GatherArgs& a, const GatherPlan& pl) {
   return stream_ok(a, pl) && (K == 64 || K == 128) && !a.stats && (uintptr_t)a.x % 16 == 0 &&
          (int64_t)a.ph[0].Q * a.P * 4 <= kMaxBufBytes;
 }
-// The split tile has no BN loader: its plans run as tile 2 there.
 static GatherPlan eff_plan(const GatherArgs& a, GatherPlan pl) {
-  if (gtile(pl.tile).split && a.bn_mean) pl.tile = 2;
   if (gtile(pl.tile).stream == 2 && !wst_ok(a, pl)) pl.tile = pl.tile - pl.tile % kNGather + kStreamTile;
   if (gtile(pl.tile).stream && !stream_ok(a, pl)) pl.tile = pl.tile - pl.tile % kNGather + 2;
   return pl;
@@ -3498,7 +3496,19 @@ static GatherPlan fwd_plan(const omt_conv_geo* g) {
   const bool have = cached_plan(OMT_DIR_FWD, g, &cp);
   return gather_plan(g->co, g->n * g->oh * g->ow, g->ci * g->ks * g->ks, 1, have ? &cp : nullptr);
 }
-// Forward workspace: the tap-major filter (when the plan's K-block divides C and ks > 1), or the split tile's packed
+// The BN loader's plan where the forward's is the split tile, which has no such loader: by rows, reduction and grid, the
+// fp32 tile that was the fastest in the loader (us; in brackets the fp32 plan tuned without the loader, then the split
+// tile's plan run as tile 2): 1x1 128 -> 512 channels at 28x28, batch 256: tile 1 408 (547, 547); 512 -> 128: 403 (437,
+// 513); 2048 -> 512 at 7x7: tile 8 507 (762, 669); 512 -> 512 stride 2 at 28x28, batch 32: tile 5 84 (86, 106); 3x3 64 ->
+// 64 at 56x56: tile 5 993 (992, 1108); 128 -> 32 at 28x28: tile 15 454 (454, -); 512 -> 512 at 7x7: tile 5 in four slices
+// 1028 (1031, 1494).
+static GatherPlan loader_plan(int64_t P, int64_t Q, int64_t K) {
+  const bool deep = K > 2048 && cdiv(P, 64) * cdiv(Q, 64) < 16 * kCUs;  // four slices even out a few rounds
+  const int tile = deep ? 5 : P <= 32 ? 15 : P <= 64 ? 5 : K >= 1024 ? 8 : cdiv(P, 128) * cdiv(Q, 128) < kCUs ? 5 : 1;
+  const omt_conv_plan p{tile, deep ? 4 : 1};
+  return gather_plan(P, Q, K, 1, &p);
+}
+// Forward workspace (that of the BN loader's plan, where it differs, if larger): the tap-major filter (when the plan's K-block divides C and ks > 1), or the split tile's packed
 // filter, then, 256-byte aligned, the split-K partials.
 static size_t fwd_pack_bytes(const omt_conv_geo* g, const GatherPlan& pl) {
   if (gtile(pl.tile).split) {
@@ -3513,10 +3523,16 @@ static size_t fwd_pack_bytes(const omt_conv_geo* g, const GatherPlan& pl) {
   return (size_t)(g->co * g->ci * g->ks * g->ks) * sizeof(float);
 }
 
-static size_t fwd_workspace_one(const omt_conv_geo* g) {
-  const GatherPlan pl = fwd_plan(g);
+static GatherPlan fwd_loader_plan(const omt_conv_geo* g, const GatherPlan& pl) {
+  return gtile(pl.tile).split ? loader_plan(g->co, g->n * g->oh * g->ow, g->ci * g->ks * g->ks) : pl;
+}
+static size_t fwd_plan_workspace(const omt_conv_geo* g, const GatherPlan& pl) {
   const size_t part = pl.slices > 1 ? (size_t)(pl.slices * g->n * g->co * g->oh * g->ow) * sizeof(float) : 0;
   return part ? align256(fwd_pack_bytes(g, pl)) + part : fwd_pack_bytes(g, pl);
+}
+static size_t fwd_workspace_one(const omt_conv_geo* g) {
+  const GatherPlan pl = fwd_plan(g);
+  return std::max(fwd_plan_workspace(g, pl), fwd_plan_workspace(g, fwd_loader_plan(g, pl)));
 }
 
 OMT_EXPORT size_t omt_conv_fwd_workspace(const omt_conv_geo* g) {
@@ -3538,13 +3554,13 @@ static int conv_fwd_one(const omt_conv_geo* g, const float* x, const float* w, c
   if (need && (!workspace || workspace_bytes < need))
     return fail(OMT_INVALID, "omt_conv_fwd: workspace of %zu bytes needed", need);
   hipStream_t s = stream_of(stream);
-  const GatherPlan pl = fwd_plan(g);
+  const GatherPlan plan = fwd_plan(g), pl = bn ? fwd_loader_plan(g, plan) : plan;
   if (stats && pl.slices > 1) return fail(OMT_UNSUPPORTED, "omt_conv_fwd_stats: the plan splits K");
   GatherArgs a{};
   a.x = x;
   a.w = w;
   // tap-major order: re-pack the filter to [co][ky][kx][ci] (1x1 filters already are)
-  const bool split = !bn && gtile(pl.tile).split;
+  const bool split = gtile(pl.tile).split;
   if (!bn && !split && fwd_pack_bytes(g, pl)) {
     const int total = (int)(g->co * g->ci * g->ks * g->ks);
     hipLaunchKernelGGL(pack_tapmajor_kernel, dim3(grid1d(total, 256, 4096)), dim3(256), 0, s, w, (float*)workspace,

@@ -479,3 +479,22 @@ def test_split_grad_weight_index_and_untuned_plans():
             assert plan(WN, g) == want
     finally:
         L.omt_conv_clear_plans()
+
+
+def test_forward_workspace_holds_the_bn_loaders_plan():
+    """A forward whose plan is the split tile runs a call with the BN loader on an fp32 tile, over a deep reduction and
+    a grid of few rounds in four K slices: the workspace holds those partials too (and the loader's plan alone where K
+    is short)."""
+    from omarchy_mac_torch import _lib
+    L = _lib.L
+    L.omt_conv_clear_plans()
+    try:
+        for n, ci, co, h, ks, parts in ((256, 512, 512, 7, 3, 4), (256, 128, 512, 28, 1, 0), (1024, 512, 512, 14, 3, 0)):
+            g = _lib.conv_geo(n, ci, co, h, h, ks, 1, ks // 2)
+            assert L.omt_conv_set_plan(_lib.OMT_DIR_FWD, ctypes.byref(g),
+                                       ctypes.byref(_lib.ConvPlan(_lib.TILE_SPLIT, 1))) == _lib.OMT_OK
+            pack = co * ci * ks * ks
+            want = 4 * pack + parts * n * co * h * h * 4 if parts else 6 * pack
+            assert L.omt_conv_fwd_workspace(ctypes.byref(g)) == want, (n, ci, co)
+    finally:
+        L.omt_conv_clear_plans()

@@ -319,6 +319,28 @@ def test_the_worst_operands_of_the_kept_products(cuda, ops):
         ops.clear_conv_plans()
 
 
+@pytest.mark.parametrize("shape", [(2, 32, 31, 9, 9, 3, 1, 1), (2, 24, 64, 9, 8, 3, 2, 1), (2, 1030, 70, 5, 7, 1, 1, 0),
+                                   (2, 232, 72, 6, 6, 3, 1, 1), (1, 40, 130, 9, 9, 1, 1, 0), (3, 16, 256, 80, 80, 1, 1, 0)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_bn_loader_beside_a_split_plan(cuda, ops, shape):
+    """Each fp32 tile that the BN loader runs where the plan is the split tile (by rows, reduction and grid), with bias
+    and ReLU, against the oracle: both within K 2^-24 of the sum of magnitudes and the rounding of the loader."""
+    n, ci, co, h, w, ks, s, p = shape
+    rng = np.random.default_rng(sum(shape))
+    x, wt, b = rnd(rng, n, ci, h, w), rnd(rng, co, ci, ks, ks, scale=(ci * ks * ks) ** -0.5), rnd(rng, co)
+    bn = [rnd(rng, ci, scale=0.2), np.abs(rnd(rng, ci)) + np.float32(0.5), rnd(rng, ci), rnd(rng, ci)]
+    c = [v.reshape(1, -1, 1, 1).astype(np.float64) for v in bn]
+    z = np.maximum((x - c[0]) / np.sqrt(c[1] + 1e-5) * c[2] + c[3], 0).astype(np.float32)
+    ref = np.maximum(orc.conv_fwd(z, wt, b, s, p), 0)
+    dev = [torch.from_numpy(v).to(cuda) for v in (x, wt, b, *bn)]
+    try:
+        ops.set_conv_plan("fwd", x.shape, wt.shape, s, p, SPLIT, 1)
+        y = ops.conv2d(dev[0], dev[1], dev[2], s, p, relu=True, bn=dev[3:]).cpu().numpy()
+        assert orc.rel_l2(y, ref) <= 1e-5  # up to 2310 products' roundings and five of the loader's, random signs
+    finally:
+        ops.clear_conv_plans()
+
+
 def test_a_workgroup_redoes_all_its_tiles(cuda, ops):
     """283 tiles on 256 CUs: a NaN in one of them has its workgroup compute all its tiles again in fp32."""
     rng = np.random.default_rng(11)

@@ -268,6 +268,8 @@ int omt_conv_set_plan(int dir, const omt_conv_geo* g, const omt_conv_plan* plan)
 int omt_conv_plan_count(void);
 int omt_conv_plan_entry(int i, int* dir, omt_conv_geo* g, omt_conv_plan* plan);
 void omt_conv_clear_plans(void);
+/* 1 if OMT_TILE_SPLIT is among the plans that omt_conv_autotune times with all tiles, else 0. */
+int omt_conv_split_candidate(int dir, const omt_conv_geo* g);
 int omt_conv_autotune(int dir, const omt_conv_geo* g, int max_tiles, void* stream, omt_conv_plan* best);
 /* Tunes the grad-input and grad-weight plans together for omt_conv_bwd: the pair tuned one direction at a time
  * (omt_conv_autotune of each) against every pair of candidates that shares a launch, timed through omt_conv_bwd;

@@ -4868,6 +4868,13 @@ int refuse_capture(hipStream_t s, const char* what) {
 
 }  // namespace
 
+OMT_EXPORT int omt_conv_split_candidate(int dir, const omt_conv_geo* g) {
+  omt_conv_geo tmp;
+  if (plan_args_ok(dir, g, tmp, "omt_conv_split_candidate")) return 0;
+  const std::vector<omt_conv_plan> cands = tune_candidates(dir, g, num_tiles(dir));
+  return std::any_of(cands.begin(), cands.end(), [](const omt_conv_plan& c) { return c.tile == OMT_TILE_SPLIT; });
+}
+
 OMT_EXPORT int omt_conv_autotune(int dir, const omt_conv_geo* g, int max_tiles, void* stream, omt_conv_plan* best) {
   omt_conv_geo tmp;
   if (int st = plan_args_ok(dir, g, tmp, "omt_conv_autotune")) return st;

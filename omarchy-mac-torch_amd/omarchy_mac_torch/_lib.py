@@ -178,6 +178,7 @@ SIGNATURES = {
                                  ctypes.POINTER(SliceSum), VP]),
     "omt_slice_sums": (I32, [ctypes.POINTER(SliceSum), I32, VP]),
     "omt_conv_num_tiles": (I32, [I32]),
+    "omt_conv_split_candidate": (I32, [I32, G]),
     "omt_conv_get_plan": (I32, [I32, G, PL, ctypes.POINTER(I32)]),
     "omt_conv_set_plan": (I32, [I32, G, PL]),
     "omt_conv_plan_count": (I32, []),

@@ -9,6 +9,7 @@ required: a missing build raises ImportError instead of running anything elsewhe
 import atexit
 import collections.abc
 import contextlib
+import ctypes
 import functools
 import json
 import os
@@ -200,6 +201,9 @@ FALLBACKS = _FallbackView()
 # index this library's gfx950 tile tables (the file name carries the gather table's size and its revision, so that
 # plans chosen among another table's kernels are not read), so the file is not the reference's, whose entries name its
 # own tiles and a split-K multiplier.
+# A file written before the split-bf16 tiles (LEGACY_TUNE_FILE) still holds for layers that they are no candidate for:
+# the fp32 tiles' indices are the same.
+LEGACY_TUNE_FILE = os.path.expanduser("~/.cache/omarchy-mac-torch/tuning-gfx950-t20.json")
 TUNE_FILE = os.environ.get(
     "OMARCHY_MAC_TORCH_TUNE_FILE",
     os.path.expanduser(f"~/.cache/omarchy-mac-torch/tuning-gfx950-t{_lib.L.omt_conv_num_tiles(_lib.OMT_DIR_FWD) // 3}r3.json"))
@@ -222,8 +226,8 @@ class TuningStore:
             return {}
         return data if isinstance(data, dict) else {}
 
-    def load(self):
-        """Returns the number of entries the plan cache accepted."""
+    def load(self, keep=lambda direction, geo: True):
+        """Returns the number of entries the plan cache accepted, of those that `keep` keeps."""
         good, self.skipped = {}, 0
         for key, val in self._read().items():
             fields = key.split(",") if isinstance(key, str) else []
@@ -232,7 +236,13 @@ class TuningStore:
                     or not all(isinstance(v, int) and not isinstance(v, bool) for v in plan)):
                 self.skipped += 1
                 continue
-            good[key] = (plan[0], plan[1])
+            try:
+                direction, *geo = (int(f) for f in fields)
+            except ValueError:  # "--1", digits of another script
+                self.skipped += 1
+                continue
+            if keep(direction, _lib.ConvGeo(*geo)):
+                good[key] = (plan[0], plan[1])
         accepted = core.tune_load(good) if good else 0
         self.skipped += len(good) - accepted
         return accepted
@@ -262,5 +272,7 @@ def _save_at_exit(store):
 
 if core.tuning():
     _store = TuningStore()
+    if "OMARCHY_MAC_TORCH_TUNE_FILE" not in os.environ:
+        TuningStore(LEGACY_TUNE_FILE).load(lambda d, g: not _lib.L.omt_conv_split_candidate(d, ctypes.byref(g)))
     _store.load()
     atexit.register(_save_at_exit, _store)

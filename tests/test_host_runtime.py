@@ -92,6 +92,28 @@ def test_tuning_file_skips_malformed_entries(core, tmp_path):
     assert set(json.loads(path.read_text())) == {f"0,{GEO}", f"2,{GEO}"}
 
 
+def test_plans_saved_before_the_split_tiles(tmp_path):
+    """The default plan file's predecessor is read for layers below the split tiles' range; a layer that they are a
+    candidate for is tuned again, and the current file's entries win."""
+    cache = tmp_path / ".cache" / "omarchy-mac-torch"
+    cache.mkdir(parents=True)
+    small, big, both = "32,64,64,16,16,16,16,3,1,1", "256,64,64,56,56,56,56,3,1,1", "32,128,128,8,8,8,8,3,1,1"
+    (cache / "tuning-gfx950-t20.json").write_text(json.dumps(
+        {f"{d},{geo}": [1, 2] for d in range(6) for geo in (small, big, both)} |
+        {"0,bad": [1, 1], f"0,--{small}": [1, 1], f"²,{small}": [1, 1]}))
+    child = ("import json; from omarchy_mac_torch import native; "
+             "print(native.TUNE_FILE); print(json.dumps(native.core.tune_dump()))")
+    env = {k: v for k, v in os.environ.items() if not k.startswith("OMARCHY_MAC_TORCH")} | {
+        "HOME": str(tmp_path), "PYTHONPATH": str(pathlib.Path(__file__).resolve().parent.parent / "omarchy-mac-torch_amd")}
+    for want in ([1, 2], [5, 3]):
+        r = subprocess.run([sys.executable, "-c", child], capture_output=True, text=True, env=env, timeout=300)
+        assert r.returncode == 0, r.stderr
+        path, dump = r.stdout.strip().splitlines()[-2:]
+        assert json.loads(dump) == {f"{d},{geo}": (want if (d, geo) == (0, both) else [1, 2])
+                                    for d in range(6) for geo in (small, both)}
+        pathlib.Path(path).write_text(json.dumps({f"0,{both}": [5, 3]}))
+
+
 def test_tuning_file_save_merges_and_the_cache_wins(core, tmp_path):
     from omarchy_mac_torch import native
     path = tmp_path / "sub" / "tune.json"

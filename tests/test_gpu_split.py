@@ -341,6 +341,34 @@ def test_bn_loader_beside_a_split_plan(cuda, ops, shape):
         ops.clear_conv_plans()
 
 
+@pytest.mark.parametrize("shape", [(2, 64, 64, 8, 8, 3, 1, 1), (2, 48, 64, 8, 8, 3, 1, 1), (2, 64, 64, 9, 9, 3, 2, 1)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_a_redone_tile_goes_through_every_epilogue(cuda, ops, shape):
+    """Tiles computed again in fp32 (tiny filter, huge source): three K slices' partials, bias and ReLU, and epilogue
+    statistics are the fp32 tile's, to the bit."""
+    n, ci, co, h, w, ks, s, p = shape
+    rng = np.random.default_rng(sum(shape))
+    x, wt, b = rnd(rng, n, ci, h, w) * np.float32(2.0 ** 100), rnd(rng, co, ci, ks, ks) * np.float32(2.0 ** -110), rnd(rng, co)
+    gy = rnd(rng, n, co, (h + 2 * p - ks) // s + 1, (w + 2 * p - ks) // s + 1) * np.float32(2.0 ** 100)
+    t = [torch.from_numpy(v).to(cuda) for v in (x, wt, b)]
+    tc = [v.contiguous(memory_format=_CL) for v in t[:2]] + t[2:]
+    try:
+        if ci == 64:  # both tiles' slices end at the same K
+            for d in ("fwd", "dgrad", "fwd_nhwc", "dgrad_nhwc"):
+                got = [run_dir(ops, d, [x, wt, gy], s, p, tile, 3) for tile in (SPLIT, FP32)]
+                assert np.array_equal(*got), d
+        got = []
+        for tile in (SPLIT, FP32):
+            for d in ("fwd", "fwd_nhwc"):
+                ops.set_conv_plan(d, x.shape, wt.shape, s, p, tile, 1)
+            y, st, groups = ops.conv2d_stats(t[0], t[1], s, p)
+            got.append([ops.conv2d(*t, s, p, relu=True), ops.conv2d_nhwc(*tc, s, p, relu=True), y, st[:, :groups]])
+        for u, v in zip(*got):
+            assert torch.equal(u, v) and float(u.abs().max()) > 0
+    finally:
+        ops.clear_conv_plans()
+
+
 def test_a_workgroup_redoes_all_its_tiles(cuda, ops):
     """283 tiles on 256 CUs: a NaN in one of them has its workgroup compute all its tiles again in fp32."""
     rng = np.random.default_rng(11)

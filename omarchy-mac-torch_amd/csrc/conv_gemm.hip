@@ -2951,13 +2951,18 @@ static int tile_bp(const Tile& tl, int64_t P) { return tl.split ? split_bp(P) : 
 // An upper bound on the bytes of the split tile's packed filter (z phases of at most K); past 2 GiB its plans run as
 // tile 2.
 static bool split_fits(int64_t P, int64_t K, int64_t z) { return z * (P + 128) * (K + 32) * 6 <= kMaxBufBytes; }
-// Whether the split tile is among the plans to choose from: 2^30 multiply-adds or more (z phases of P x Q x K). Below
-// that the smaller fp32 tiles fill the GPU better and its filter pack is a launch too many: 64 channels over 32 images
-// of 16 x 16 (0.3 x 2^30) take 15 us on the tuned fp32 tile and 28 on the split tile in its best K split; 256 over 64
-// images of 14 x 14 (6.9 x 2^30) 167 and 114, 64 over 64 images of 28 x 28 (1.7 x 2^30) 50 and 40.
-static bool split_pays(int64_t P, int64_t Q, int64_t K, int64_t z) {
-  return split_fits(P, K, z) && P * Q * K * z >= ((int64_t)1 << 30);
+// Whether the tuner times the split tile: from 2^30 multiply-adds on (z phases of P x Q x K). Below, the smaller fp32
+// tiles fill the GPU better and its filter pack is a launch too many. The fastest fp32 plan of all and the split tile's
+// best K split, us of a call in a replayed graph, at 0.3, 0.5, 0.7, 1.0, 1.5 and 2.0 times 2^30, forward: 3x3 64 channels at
+// 28x28 19/29, 19/32, 25/32, 29/32, 39/34, 49/36; 3x3 256 at 14x14 26/45, 27/48, 33/50, 39/51, 50/51, 59/55; 1x1 128 ->
+// 512 at 28x28 13/23, 17/24, 22/26, 29/41, 37/40, 49/54 (grad input and channels last alike).
+// The estimate of an untuned call takes it from 2^33 on: there every layer measured was at least as fast as on the fp32
+// plan estimated, 1.01-1.7 times; at 2^32 one was at 0.89 (channels-last grad input of 1x1 64 -> 256 at 56x56), at
+// 2 x 2^30 several at 0.8-0.95, whose grids leave a second round nearly empty.
+static bool split_pays(int64_t P, int64_t Q, int64_t K, int64_t z, int log2 = 30) {
+  return split_fits(P, K, z) && P * Q * K * z >= ((int64_t)1 << log2);
 }
+constexpr int kSplitUntuned = 33;
 
 static const Tile kWgradTiles[] = {
     {64, 128, 32, 64, 1.00f}, {128, 64, 32, 64, 1.00f}, {64, 64, 32, 32, 0.85f}, {32, 128, 16, 64, 0.85f},
@@ -2983,7 +2988,11 @@ static int wgrad_split_shape(int64_t P, int64_t Q) {
   }
   return best;
 }
-static bool wgrad_split_pays(int64_t P, int64_t Q, int64_t K) { return P * Q * K >= ((int64_t)1 << 30); }
+// Whether the tuner times it, and whether an untuned call takes it, from 2^33 multiply-adds on, or, channels last, 2^31
+// (against the fp32 plan estimated: 0.96-2.2 times as fast at 2^32, the slowest 3x3 64 channels at 28x28, 1.06-2.5 at 2^33;
+// channels last 0.97-1.26 at 2^30, 1.1-1.5 at 2^31).
+static bool wgrad_split_pays(int64_t P, int64_t Q, int64_t K, int log2 = 30) { return P * Q * K >= ((int64_t)1 << log2); }
+static int wgrad_split_untuned(int dir) { return dir == OMT_DIR_WGRAD_NHWC ? 31 : kSplitUntuned; }
 
 template <int MODE, bool BN>
 static void gather_dispatch(int ti, const GatherArgs& a, dim3 grid, hipStream_t s) {
@@ -3150,7 +3159,7 @@ static GatherPlan gather_plan(int64_t P, int64_t Q, int64_t K, int64_t z, const 
     const Tile& tl = gtile(ti);
     if (tl.stream) continue;  // chosen by tuning only
     if (nhwc_c && !nhwc_tile_ok(ti, nhwc_c)) continue;
-    if (tl.split && !split_pays(P, Q, kk, z)) continue;
+    if (tl.split && !split_pays(P, Q, kk, z, kSplitUntuned)) continue;
     const int bp = tile_bp(tl, P);
     const int64_t tiles = cdiv(P, bp) * cdiv(Q, tl.bq) * z, nkb = cdiv(kk, tl.bk);
     for (int sc : kSliceChoices) {
@@ -3406,7 +3415,7 @@ static WgradPlan wgrad_plan(const omt_conv_geo* g, int dir = OMT_DIR_WGRAD) {
     ti = cp.tile == OMT_TILE_SPLIT && !wgrad_split_ok(dir, g) ? 2 : cp.tile;
     slices = std::max<int64_t>(1, std::min<int64_t>(cp.slices, cdiv(K, 64)));
   } else {
-    ti = wgrad_split_pays(P, Q, K) && wgrad_split_ok(dir, g) ? OMT_TILE_SPLIT : pick_tile(kWgradTiles, P, Q, 1, kCUs * 2);
+    ti = wgrad_split_pays(P, Q, K, wgrad_split_untuned(dir)) && wgrad_split_ok(dir, g) ? OMT_TILE_SPLIT : pick_tile(kWgradTiles, P, Q, 1, kCUs * 2);
     slices = wgrad_model_slices(g, ti);
   }
   const int64_t kslice = cdiv(cdiv(K, slices), 64) * 64;

@@ -451,7 +451,7 @@ def test_the_split_tile_has_an_index_of_its_own():
 def test_split_grad_weight_index_and_untuned_plans():
     """The four fp32 grad-weight tiles keep indices 0-3 in both memory formats, OMT_TILE_SPLIT is a plan of both
     (channels last with input channels that are no multiple of 8 it runs as tile 2), and an untuned plan is the split
-    tile from 2^30 multiply-adds on and never below, in every direction."""
+    tile from 2^33 multiply-adds on (channels-last grad weight 2^31) and not below, where the tuner alone picks it."""
     from omarchy_mac_torch import _lib
     L = _lib.L
     W, WN = _lib.OMT_DIR_WGRAD, _lib.OMT_DIR_WGRAD_NHWC
@@ -473,6 +473,9 @@ def test_split_grad_weight_index_and_untuned_plans():
         assert plan(WN, g) == plan(W, g) == 3  # 32 rows, 61952 columns: the fp32 32 x 128 tile
         big = _lib.conv_geo(256, 64, 64, 56, 56, 3, 1, 1)  # 28 x 2^30
         assert [plan(d, big) for d in range(6)] == [_lib.TILE_SPLIT] * 6
+        mid = _lib.conv_geo(32, 64, 64, 56, 56, 3, 1, 1)   # 3.4 x 2^30
+        assert all(L.omt_conv_split_candidate(d, ctypes.byref(mid)) for d in range(6))
+        assert [plan(d, mid) == _lib.TILE_SPLIT for d in range(6)] == [False] * 5 + [True]
         for ci, want in ((64, _lib.TILE_SPLIT), (60, 2)):
             g = _lib.conv_geo(2, ci, 64, 14, 14, 3, 1, 1)
             assert L.omt_conv_set_plan(WN, ctypes.byref(g), ctypes.byref(_lib.ConvPlan(_lib.TILE_SPLIT, 2))) == _lib.OMT_OK

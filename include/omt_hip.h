@@ -141,7 +141,7 @@ void omt_kernel_stats_reset(int what);
 int omt_kernel_stat_count(void);
 int omt_kernel_stat_entry(int i, const char** name, int64_t* launches, double* ms);
 
-/* ---- dense convolution (implicit GEMM on MFMA: fp32, or fp32 products as six exact bf16 ones) ---------------- */
+/* ---- dense convolution (implicit GEMM on MFMA: fp32, or fp32 products as six bf16 ones of nine) ---------------- */
 
 /* Forward: y[n][co][oh][ow] = sum_{ci,ky,kx} x[n][ci][oy*s+ky-p][ox*s+kx-p] * w[co][ci][ky][kx], then
  * + bias[co] (epilogue & OMT_EPI_BIAS) and ReLU (epilogue & OMT_EPI_RELU).
